@@ -13,6 +13,7 @@
 #include "galerkin.hpp"
 #include "host_setup.hpp"
 #include "kernels.hpp"
+#include "sweep_group.hpp"
 
 namespace unap_hip {
 
@@ -84,8 +85,10 @@ struct Ctx {
     DBuf<double> partials;
     DBuf<KState> scratchState;  // for standalone calls (eigen estimate, precond apply)
     static Ctx& get();
+    DBuf<GroupSync> group;             // meeting place of the group sweeps (sweep_group.hpp)
+    volatile int* groupFail = nullptr;  // pinned host word: one of their waits gave up
     static Ctx* peek();  // the context if it exists (creating it allocates)
-    void sync() { UH_CHECK(hipStreamSynchronize(stream)); }
+    void sync();
 };
 
 struct Launch {
@@ -188,6 +191,36 @@ __global__ void kBuildBwdCopy(DMat<T> A, const int* __restrict__ bwdRows, const 
     }
 }
 
+// Packed table of the group sweeps (sweep_group.hpp): groups of a wavefront's
+// rows, level by level.  The groups are made once; the entries are refilled
+// from the matrix after its values change, into the same buffers.
+struct GroupTab {
+    int rows = 0;  // rows a group
+    int ng = 0;
+    bool filled = false;
+    DBuf<int2> grp;    // first schedule position and row count of a group
+    DBuf<int> grp0;    // groups before each level
+    DBuf<int> grpOvf;  // a group's first chunk in the overflow table
+    DBuf<uint4> tab, ovf;
+    // levels of one or two schedules (bounds s0, then s1), groups of rw rows
+    void plan(const std::vector<int>& s0, const std::vector<int>* s1, int rw, std::vector<int2>& g, hipStream_t s) {
+        std::vector<int> first(1, 0);
+        g.clear();
+        for (const std::vector<int>* st : {&s0, s1}) {
+            if (!st) continue;
+            for (size_t k = 0; k + 1 < st->size(); ++k) {
+                for (int q = (*st)[k]; q < (*st)[k + 1]; q += rw) g.push_back({q, std::min(rw, (*st)[k + 1] - q)});
+                first.push_back((int)g.size());
+            }
+        }
+        rows = rw;
+        ng = (int)g.size();
+        grp.upload(g, s);
+        grp0.upload(first, s);
+        UH_CHECK(hipStreamSynchronize(s));
+    }
+};
+
 // Device copy of one matrix in precision T.
 template <typename T>
 struct DevMatrix {
@@ -214,6 +247,73 @@ struct DevMatrix {
     DBuf<uint32_t> bwdInfo;
     DBuf<int> bwdCol;
     DBuf<T> bwdVal;
+    GroupTab gsTab, luTab;  // made on first use
+
+    // Lanes a row of the Gauss-Seidel table: kGsS entries a lane cover the
+    // average row and most of the spread.
+    int gsLanes() const { return entriesPerRow <= 7.0 ? 2 : (entriesPerRow <= 12.5 ? 4 : 8); }
+    // The tables need the level-major order (position = row).
+    const GroupTab& gsTable(hipStream_t s) {
+        GroupTab& t = gsTab;
+        const int lpr = gsLanes();
+        if (!t.tab.p) {
+            std::vector<int2> g;
+            t.plan(fwdStartH, nullptr, 64 / lpr, g, s);
+            std::vector<uint32_t> info(n);
+            UH_CHECK(hipMemcpyAsync(info.data(), rowInfo.get(), sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
+            UH_CHECK(hipStreamSynchronize(s));
+            const int chunk = lpr * kGsS;
+            std::vector<int> at(t.ng, 0);
+            int next = 0;
+            for (int k = 0; k < t.ng; ++k) {
+                int most = 0;
+                for (int q = g[k].x; q < g[k].x + g[k].y; ++q) most = std::max(most, (int)(info[q] & 0xffffu));
+                at[k] = next;
+                if (most > chunk) next += (most - 1) / chunk;
+            }
+            t.grpOvf.upload(at, s);
+            UH_CHECK(hipStreamSynchronize(s));
+            t.tab.alloc((size_t)t.ng * GroupPack<T>::kGs * 64);
+            t.ovf.alloc((size_t)std::max(next, 1) * GroupPack<T>::kOvf * 64);
+            t.filled = false;
+        }
+        if (!t.filled) {
+            const int grid = (t.ng + 3) / 4;
+            auto fill = [&](auto kernel) {
+                kernel<<<grid, 256, 0, s>>>(view(), t.grp.get(), t.grpOvf.get(), t.ng, t.tab.get(), t.ovf.get());
+            };
+            if (lpr == 2)
+                fill(kPackGs<2, T>);
+            else if (lpr == 4)
+                fill(kPackGs<4, T>);
+            else
+                fill(kPackGs<8, T>);
+            UH_LAUNCHED();
+            t.filled = true;
+        }
+        return t;
+    }
+    const GroupTab& luTable(hipStream_t s) {
+        GroupTab& t = luTab;
+        if (!t.tab.p) {
+            std::vector<int2> g;
+            t.plan(fwdStartH, &bwdStartH, 64, g, s);
+            t.tab.alloc((size_t)t.ng * GroupPack<T>::kLu * 64);
+            t.filled = false;
+        }
+        if (!t.filled) {
+            int nf = 0;  // groups of the forward levels
+            for (size_t k = 0; k + 1 < fwdStartH.size(); ++k) nf += (fwdStartH[k + 1] - fwdStartH[k] + 63) / 64;
+            const int nb = t.ng - nf;
+            kPackLu<T><<<(nf + 3) / 4, 256, 0, s>>>(view(), nullptr, 1, t.grp.get(), nf, t.tab.get());
+            UH_LAUNCHED();
+            kPackLu<T><<<(nb + 3) / 4, 256, 0, s>>>(bwdView(s), bwdRows.get(), 0, t.grp.get() + nf, nb,
+                                                    t.tab.get() + (size_t)nf * GroupPack<T>::kLu * 64);
+            UH_LAUNCHED();
+            t.filled = true;
+        }
+        return t;
+    }
 
     DMat<T> view() const { return {n, sliceStart.get(), rowInfo.get(), col.get(), val.get(), diag.get()}; }
     DMat<T> viewU() const {
@@ -315,6 +415,7 @@ struct DevMatrix {
         }
         valU.release();
         bwdVal.release();  // rebuilt from the new values on the next backward sweep
+        gsTab.filled = luTab.filled = false;
     }
     // Addressing, schedules and the backward-copy structure; no values.
     void buildStructure(const Layout& L, hipStream_t s) {
@@ -366,6 +467,7 @@ struct DevMatrix {
         fillDiagFrom(A, s);
         valU.release();
         bwdVal.release();  // rebuilt from the new values on the next backward sweep
+        gsTab.filled = luTab.filled = false;
         if (hadU) buildValU(A, L, s);
     }
 };

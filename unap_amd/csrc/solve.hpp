@@ -179,11 +179,65 @@ void runSchedule(SweepArgs<T, TV> a, const std::vector<int>& levStartH, int maxR
     }
 }
 
+// Sweeps by a group of workgroups on one XCD (sweep_group.hpp).  A level costs
+// the group about 0.9 us plus its share of the packed table at the 0.5 TB/s one
+// XCD draws; launched, it costs about 5 us plus the same at the whole chip's
+// rate (kSweepLevel / kGsLevelLanes), or 1-3 us in the one-workgroup tail.  The
+// lines below are where the two meet, in table bytes a level (MI355X): DIC
+// FP32 224k rows (0.68 MB) 115 against 155 us an application, DILU FP32 466k
+// rows (1.57 MB) 195 against 155; Gauss-Seidel FP64 on 105k rows of 17 entries
+// (1.3 MB) 3.4 against 5.5 us a level, on 220k of 15 (3.2 MB) 7.1 against 6.4.
+constexpr double kGroupLuBytes = 0.9e6, kGroupGsBytes = 1.6e6;
+constexpr int kGroupCUs = 32;  // workgroups a group on one XCD has when all its CUs are free
+
+// The sweep schedules the packed tables serve: level-major order (position =
+// row), level bounds that fit the launch's LDS list.
+template <typename T>
+bool groupSchedule(const DevMatrix<T>& M, size_t levels) {
+    return !M.fwdRows.p && levels <= (size_t)kGroupLevels;
+}
+template <typename T>
+bool groupGsFits(const DevMatrix<T>& M) {
+    const size_t nl = M.fwdStartH.size() - 1;
+    return groupSchedule(M, nl) && 16.0 * GroupPack<T>::kGs * M.gsLanes() * M.n <= kGroupGsBytes * (double)nl;
+}
+template <typename T>
+bool groupLuFits(const DevMatrix<T>& M) {
+    const size_t nl = M.fwdStartH.size() - 1;
+    return groupSchedule(M, nl + M.bwdStartH.size() - 1) &&
+           16.0 * GroupPack<T>::kLu * M.n <= kGroupLuBytes * (double)nl;
+}
+inline GroupCtl groupCtl() {
+    Ctx& c = Ctx::get();
+    return {c.group.get(), const_cast<int*>(c.groupFail), kGroupCUs, 1};
+}
+
+template <typename T>
+void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, Skip sk) {
+    Ctx& cx = Ctx::get();
+    const GroupTab& t = M.gsTable(cx.stream);
+    const GroupGs<T> g{t.tab.get(), t.ovf.get(), t.grp0.get(), M.fwdStart.get(), (int)M.fwdStartH.size() - 1, nSweeps,
+                       x, b};
+    const GroupCtl c = groupCtl();
+    const int grid = 8 * c.expect, lpr = M.gsLanes();  // workgroups go to the eight XCDs in turn
+    if (lpr == 2)
+        kGroupGs<true, 2><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
+    else if (lpr == 4)
+        kGroupGs<true, 4><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
+    else
+        kGroupGs<true, 8><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
+    UH_LAUNCHED();
+}
+
 // Gauss-Seidel smoothing, nSweeps forward sweeps (lduGaussSeidelSmoother.cpp:40-79).
 template <typename T>
 void gsSmooth(DevMatrix<T>& M, T* x, const T* b, int nSweeps, Skip sk) {
     if (!M.sweepable) throw Error(-3, "Gauss-Seidel needs faces sorted by owner with owner < neighbour");
     SweepArgs<T, T> a{M.view(), x, b, nullptr, M.fwdRows.p, M.fwdStart.get()};
+    if (nSweeps > 0 && groupGsFits(M)) {
+        groupGs(M, x, b, nSweeps, sk);
+        return;
+    }
     const int nl = (int)M.fwdStartH.size() - 1;
     const int maxRows = tailRows(M.entriesPerRow);  // a GS row reads all its entries
     if (tailStart(M.fwdStartH, maxRows) == 0) {
@@ -202,6 +256,20 @@ template <typename T, typename TV>
 void luSweeps(DevMatrix<T>& M, bool dic, TV* w, const TV* r, const TV* rD, Skip sk, const TV* rDpos) {
     if (!M.sweepable) throw Error(-3, "DIC/DILU needs faces sorted by owner with owner < neighbour");
     const DMat<T> Av = dic ? M.viewU() : M.view();
+    if constexpr (std::is_same<T, TV>::value) {
+        // (DIC on asymmetric storage, with its second coefficient array, and
+        // callers without the position-ordered rD run level by level)
+        if (groupLuFits(M) && !M.valU.p && rDpos) {
+            Ctx& cx = Ctx::get();
+            const GroupTab& t = M.luTable(cx.stream);
+            const GroupLu<T> g{Av, M.bwdView(cx.stream), t.tab.get(), t.grp0.get(), M.fwdStart.get(), M.bwdStart.get(),
+                               (int)M.fwdStartH.size() - 1, (int)M.bwdStartH.size() - 1, r, rD, rDpos, w};
+            const GroupCtl c = groupCtl();
+            kGroupLu<true><<<8 * c.expect, kLuThreads, 0, cx.stream>>>(g, c, sk);
+            UH_LAUNCHED();
+            return;
+        }
+    }
     SweepArgs<T, TV> f{Av, w, r, rD, M.fwdRows.p, M.fwdStart.get()};
     const int maxRows = tailRows(0.5 * M.entriesPerRow);  // one side of each row
     runSchedule<T, TV, SWEEP_FWD>(f, M.fwdStartH, maxRows, sk);

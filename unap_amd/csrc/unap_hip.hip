@@ -29,11 +29,25 @@ Ctx& Ctx::get() {
         UH_CHECK(hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking));
         n->partials.alloc((size_t)kMaxSums * kMaxBlocks);
         n->scratchState.alloc(4);
+        n->group.alloc(1);
+        UH_CHECK(hipMemsetAsync(n->group.get(), 0, sizeof(GroupSync), n->stream));
+        int* fail = nullptr;
+        UH_CHECK(hipHostMalloc((void**)&fail, sizeof(int), hipHostMallocDefault));
+        *fail = 0;
+        n->groupFail = fail;
         g_ctx = n;
     }
     return *g_ctx;
 }
 Ctx* Ctx::peek() { return g_ctx; }
+void Ctx::sync() {
+    UH_CHECK(hipStreamSynchronize(stream));
+    if (*groupFail) {
+        *groupFail = 0;
+        UH_CHECK(hipMemset(group.get(), 0, sizeof(GroupSync)));
+        throw Error(UNAP_HIP_ERR_INTERNAL, "a sweep's workgroups waited too long for one another");
+    }
+}
 
 // Pinned host mirror of one KState for flag read-back.
 static KState* hostState() {
