@@ -31,10 +31,11 @@ struct CoarseArgs {
     int serial;
 };
 
-// Sum over the workgroup, broadcast to every thread (fixed order).
+// Sum over the workgroup's first nw wavefronts, broadcast to every thread
+// (fixed order).
 template <int NS>
-__device__ __forceinline__ void wgSum(double (&v)[NS], double* red) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+__device__ __forceinline__ void wgSum(double (&v)[NS], double* red, int nw) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         double a = v[s];
@@ -42,7 +43,7 @@ __device__ __forceinline__ void wgSum(double (&v)[NS], double* red) {
         for (int o = 32; o >= 1; o >>= 1) a += __shfl_xor(a, o, 64);
         v[s] = a;
     }
-    if (lane == 0) {
+    if (lane == 0 && wave < nw) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) red[s * 16 + wave] = v[s];
     }
@@ -59,8 +60,11 @@ __device__ __forceinline__ void wgSum(double (&v)[NS], double* red) {
 // Sum term(i) over the level: tree over the workgroup, or (serial mode) one
 // thread walking the reference's cell order.  Every thread gets the totals.
 // The vectors term() reads must be complete (the caller has synchronised).
-template <int NS, class F>
+// The tree is over the first Sum threads (0: all), so that its order does not
+// depend on how many threads a kernel runs its other loops with.
+template <int NS, int Sum = 0, class F>
 __device__ __forceinline__ void wgReduce(const CoarseArgs& a, int n, F term, double (&v)[NS], double* red) {
+    const int nt = Sum ? Sum : (int)blockDim.x;
     if (a.serial) {
         if (threadIdx.x == 0) {
             double acc[NS];
@@ -83,13 +87,14 @@ __device__ __forceinline__ void wgReduce(const CoarseArgs& a, int n, F term, dou
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) v[s] = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        double t[NS];
-        term(i, t);
+    if ((int)threadIdx.x < nt)
+        for (int i = threadIdx.x; i < n; i += nt) {
+            double t[NS];
+            term(i, t);
 #pragma unroll
-        for (int s = 0; s < NS; ++s) v[s] += t[s];
-    }
-    wgSum<NS>(v, red);
+            for (int s = 0; s < NS; ++s) v[s] += t[s];
+        }
+    wgSum<NS>(v, red, nt >> 6);
 }
 
 // The coarsest matrix read in place (SELL layout in global memory).
@@ -133,7 +138,7 @@ struct CoarseLocal {
     // and coefficients, then the gathers), positions past the end re-reading
     // the batch's first entry, so a row waits on two LDS round trips a batch
     // rather than two an entry.
-    static constexpr int kLocalBatch = 8;
+    static constexpr int kLocalBatch = 4;
     template <int Op>  // 0: acc + v x;  1: acc - (rd v) x
     __device__ __forceinline__ double run(int k0, int n, int step, double acc, double rd, const double* x) const {
         for (int t0 = 0; t0 < n; t0 += kLocalBatch) {
@@ -188,9 +193,10 @@ __device__ __forceinline__ bool wgConv(double fin, double init, double tol, doub
 }
 
 // PCG + DIC (PCG.cpp:35-183) on the coarsest level; x, r, w, p in LDS.
-template <class M>
+// precond(w, r): the DIC sweeps, ending in a barrier.
+template <int Sum, class M, class Pre>
 __device__ __forceinline__ void coarsePCG(const CoarseArgs& a, const M& m, double* x, double* r, double* w,
-                                          double* p, double* red) {
+                                          double* p, double* red, Pre precond) {
     const int n = a.A.n;
     const int t = threadIdx.x, nt = blockDim.x;
     double s1[1];
@@ -201,14 +207,14 @@ __device__ __forceinline__ void coarsePCG(const CoarseArgs& a, const M& m, doubl
         p[i] = 0.0;
     }
     __syncthreads();
-    wgReduce<1>(a, n, [&](int i, double(&q)[1]) { q[0] = r[i] * r[i]; }, s1, red);
+    wgReduce<1, Sum>(a, n, [&](int i, double(&q)[1]) { q[0] = r[i] * r[i]; }, s1, red);
     const double init = sqrt(s1[0]) + kSmallD;
     double rho = 1.0e37, rhoOld;
     long long nIter = 0;
     for (;;) {
         rhoOld = rho;
-        wgPrecond(a, m, w, r);
-        wgReduce<1>(a, n, [&](int i, double(&q)[1]) { q[0] = w[i] * r[i]; }, s1, red);
+        precond();
+        wgReduce<1, Sum>(a, n, [&](int i, double(&q)[1]) { q[0] = w[i] * r[i]; }, s1, red);
         rho = s1[0];
         if (!(fabs(rho) > kSmallD)) break;
         const double beta = rho / rhoOld;
@@ -216,14 +222,14 @@ __device__ __forceinline__ void coarsePCG(const CoarseArgs& a, const M& m, doubl
         __syncthreads();
         for (int i = t; i < n; i += nt) w[i] = m.amul(i, p);
         __syncthreads();
-        wgReduce<1>(a, n, [&](int i, double(&q)[1]) { q[0] = w[i] * p[i]; }, s1, red);
+        wgReduce<1, Sum>(a, n, [&](int i, double(&q)[1]) { q[0] = w[i] * p[i]; }, s1, red);
         const double alpha = rho / s1[0];
         for (int i = t; i < n; i += nt) {
             x[i] += alpha * p[i];
             r[i] -= alpha * w[i];
         }
         __syncthreads();
-        wgReduce<1>(a, n, [&](int i, double(&q)[1]) { q[0] = r[i] * r[i]; }, s1, red);
+        wgReduce<1, Sum>(a, n, [&](int i, double(&q)[1]) { q[0] = r[i] * r[i]; }, s1, red);
         const double fin = sqrt(s1[0]) + kSmallD;
         ++nIter;
         if (!(nIter < a.maxIter)) break;
@@ -236,19 +242,113 @@ static __global__ void __launch_bounds__(1024) kCoarsePCG(CoarseArgs a, Skip sk)
     if (sk.on()) return;
     extern __shared__ double lds[];
     const int n = a.A.n;
-    coarsePCG(a, CoarseGlobal{a}, lds, lds + n, lds + 2 * n, lds + 3 * n, lds + 4 * n);
+    const CoarseGlobal m{a};
+    double *r = lds + n, *w = lds + 2 * n;
+    coarsePCG<0>(a, m, lds, r, w, lds + 3 * n, lds + 4 * n, [&] { wgPrecond(a, m, w, r); });
 }
 
 // LDS bytes of kCoarsePCGLocal for a level of n rows, nnz entries, nf / nb
 // forward / backward levels, with or without a forward row list.
 inline size_t coarseLocalBytes(int n, int nnz, int nf, int nb, bool fwdRows) {
-    const size_t d = sizeof(double) * ((size_t)nnz + 6 * (size_t)n + 64);
+    const size_t d = sizeof(double) * ((size_t)nnz + 6 * (size_t)n + 1 + 64);
     const size_t i = sizeof(int) * ((size_t)n + 1 + (fwdRows ? n : 0) + n + nf + 1 + nb + 1);
     const size_t h = sizeof(uint16_t) * ((size_t)nnz + n);
     return d + i + h + 16;
 }
 
-static __global__ void __launch_bounds__(256) kCoarsePCGLocal(CoarseArgs a, CoarseCsr c, Skip sk) {
+// One side of one row, for good in a thread's registers: the row at position
+// threadIdx.x of a sweep's schedule, its level, and rD * coefficient and
+// element of its first Cap entries (a multiple of 8).  Absent entries are 0
+// times w[n], a zero.
+template <int Cap>
+struct HeldRow {
+    int row = -1, level = -1, n = 0;
+    int lo = 1, hi = 0;  // levels of the wavefront's rows
+    double rd = 0.0, f[Cap];
+    int c[Cap];  // byte offsets of their vector elements in LDS
+};
+template <bool Fwd, int Cap>
+__device__ __forceinline__ void holdRow(const CoarseLocal& m, int nRows, int nl, int at, HeldRow<Cap>& h) {
+    const int q = (int)threadIdx.x;
+    int s0 = 0, s1 = 0;
+    if (q < nRows) {
+        h.row = Fwd ? m.frow(q) : m.brow(q);
+        int k = 0;
+        while (k + 1 < nl && q >= (Fwd ? m.fs(k + 1) : m.bs(k + 1))) ++k;
+        h.level = k;
+        s0 = m.start[h.row];
+        s1 = m.start[h.row + 1];
+        const int mid = m.mid[h.row];
+        h.n = Fwd ? mid : s1 - s0 - mid;
+        h.rd = m.rD[h.row];
+    }
+#pragma unroll
+    for (int j = 0; j < Cap; ++j) {
+        const bool on = j < h.n;
+        const int e = Fwd ? s0 + j : s1 - 1 - j;
+        h.c[j] = at + 8 * (on ? (int)m.col[e] : nRows);
+        h.f[j] = on ? h.rd * m.val[e] : 0.0;
+    }
+    // positions ascend by level, so the wavefront's first and last rows bound its levels
+    const int w0 = q & ~63, w1 = min(w0 + 63, nRows - 1);
+    if (w0 < nRows) {
+        h.lo = __builtin_amdgcn_readfirstlane(h.level);
+        h.hi = __shfl(h.level, w1 - w0, 64);
+        h.hi = __builtin_amdgcn_readfirstlane(h.hi);
+    }
+}
+// The sweep over held rows: level by level, each row in the thread that holds
+// it.  A level costs a barrier, one LDS round trip for its gathers and the
+// row's chain of subtractions (fwdRow's / bwdRow's).
+template <bool Fwd, int Cap>
+__device__ __forceinline__ void heldSweep(const CoarseLocal& m, int nRows, int nl, const HeldRow<Cap>& h,
+                                          const char* lds, double* w, const double* r) {
+    const double init = (Fwd && h.row >= 0) ? h.rd * r[h.row] : 0.0;
+    const int held = (int)blockDim.x;
+    for (int k = 0; k < nl; ++k) {
+        if (k >= h.lo && k <= h.hi) {
+            if (h.level == k) {
+                double acc = Fwd ? init : w[h.row];
+#pragma unroll
+                for (int j0 = 0; j0 < Cap; j0 += 8) {
+                    if (j0 > 0 && !__any(j0 < h.n)) break;
+                    double x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        x[j] = *reinterpret_cast<const double*>(lds + h.c[j0 + j]);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) acc = acc - h.f[j0 + j] * x[j];
+                }
+                if (h.n > Cap) {
+                    const int s0 = m.start[h.row], s1 = m.start[h.row + 1];
+                    acc = m.run<1>(Fwd ? s0 + Cap : s1 - 1 - Cap, h.n - Cap, Fwd ? 1 : -1, acc, h.rd, w);
+                }
+                w[h.row] = acc;
+            }
+        }
+        if (nRows > held) {  // positions past the threads': in place
+            const int p1 = Fwd ? m.fs(k + 1) : m.bs(k + 1);
+            for (int q = max(Fwd ? m.fs(k) : m.bs(k), held) + (int)threadIdx.x; q < p1; q += held) {
+                if (Fwd)
+                    m.fwd(m.frow(q), w, r);
+                else
+                    m.bwd(m.brow(q), w);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// kCoarsePCG with the matrix, rD, the schedule and the vectors in LDS, and
+// both sweeps' rows in registers (one row of each sweep a thread; a
+// level's rows past the threads run from LDS): 18 iterations of 60 levels on 556 rows took 1345 us with the
+// sweeps' matrix read from LDS by 256 threads (a level's row index, bounds,
+// entries and gathers one after the other), 613 us so; a 57-row one 300 and
+// 120 us.  What is left is the chain of a level: barrier, gathers,
+// subtractions, and the entries past Cap, which come from LDS.
+constexpr int kCoarseSum = 256;  // threads of the reductions' tree
+template <int Threads, int Cap>
+static __global__ void __launch_bounds__(Threads) kCoarsePCGLocal(CoarseArgs a, CoarseCsr c, Skip sk) {
     if (sk.on()) return;
     extern __shared__ double lds[];
     const int n = a.A.n, nnz = c.nnz, t = threadIdx.x, nt = blockDim.x;
@@ -257,9 +357,9 @@ static __global__ void __launch_bounds__(256) kCoarsePCGLocal(CoarseArgs a, Coar
     double* rD = diag + n;
     double* x = rD + n;
     double* r = x + n;
-    double* w = r + n;
-    double* p = w + n;
-    double* red = p + n;
+    double* p = r + n;
+    double* w = p + n;  // n + 1: w[n] is a zero
+    double* red = w + n + 1;
     int* start = reinterpret_cast<int*>(red + 64);
     int* frows = start + n + 1;
     int* brows = frows + (a.fwdRows ? n : 0);
@@ -279,12 +379,23 @@ static __global__ void __launch_bounds__(256) kCoarsePCGLocal(CoarseArgs a, Coar
         brows[i] = a.bwdRows[i];
         if (a.fwdRows) frows[i] = a.fwdRows[i];
     }
-    if (t == 0) start[n] = c.start[n];
+    if (t == 0) {
+        start[n] = c.start[n];
+        w[n] = 0.0;
+    }
     for (int k = t; k <= a.nFwd; k += nt) fs[k] = a.fwdStart[k];
     for (int k = t; k <= a.nBwd; k += nt) bs[k] = a.bwdStart[k];
     __syncthreads();
     const CoarseLocal m{val, diag, rD, start, col, mid, fs, a.fwdRows ? frows : nullptr, bs, brows};
-    coarsePCG(a, m, x, r, w, p, red);
+    HeldRow<Cap> f, b;
+    const char* base = reinterpret_cast<const char*>(lds);
+    const int at = (int)(reinterpret_cast<const char*>(w) - base);
+    holdRow<true>(m, n, a.nFwd, at, f);
+    holdRow<false>(m, n, a.nBwd, at, b);
+    coarsePCG<kCoarseSum>(a, m, x, r, w, p, red, [&] __attribute__((always_inline)) {
+        heldSweep<true>(m, n, a.nFwd, f, base, w, r);
+        heldSweep<false>(m, n, a.nBwd, b, base, w, r);
+    });
 }
 
 // PBiCGStab + DILU (PBiCGStab.cpp:45-459) on the coarsest level.

@@ -187,6 +187,15 @@ const HostLdu& AgglHost::hostLevel(int k) {
     return levels[k].A;
 }
 
+// The LDS-resident coarsest solver for n rows: as few threads as hold a row
+// each, so that the registers a thread has hold as many entries as possible.
+static std::pair<void (*)(CoarseArgs, CoarseCsr, Skip), int> coarseKernel(int n) {
+    if (n <= 256) return {kCoarsePCGLocal<256, 32>, 256};
+    if (n <= 512) return {kCoarsePCGLocal<512, 24>, 512};
+    if (n <= 768) return {kCoarsePCGLocal<768, 16>, 768};
+    return {kCoarsePCGLocal<1024, 8>, 1024};
+}
+
 template <typename T>
 void Hierarchy<T>::refresh() {
     if (valuesGen == fineObj->coeffGen) return;
@@ -329,9 +338,9 @@ void Hierarchy<T>::setupNumeric() {
             int dev = 0, optin = 0;
             UH_CHECK(hipGetDevice(&dev));
             if (hipDeviceGetAttribute(&optin, hipDeviceAttributeSharedMemPerBlockOptin, dev) != hipSuccess) optin = 0;
+            const void* kernel = (const void*)coarseKernel(n).first;
             if (bytes <= (size_t)optin &&
-                hipFuncSetAttribute((const void*)kCoarsePCGLocal, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)bytes) == hipSuccess) {
+                hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess) {
                 const Layout CLh = hostArrays(CL, c.stream);
                 std::vector<double> sv;
                 fillSellValues<double>(CLh, CA, false, sv);
@@ -454,10 +463,11 @@ void Hierarchy<T>::coarsestSolve(Skip sk) {
     a.maxIter = 100;
     a.iperm = cm->iperm.get();
     a.serial = c.serialReductions;
-    if (CA.symm && coarseLocal)
-        kCoarsePCGLocal<<<1, 256, coarseLocalLds, c.stream>>>(
-            a, CoarseCsr{csrStart.get(), csrCol.get(), csrMid.get(), csrVal.get(), (int)csrVal.n}, sk);
-    else if (CA.symm)
+    const CoarseCsr csr{csrStart.get(), csrCol.get(), csrMid.get(), csrVal.get(), (int)csrVal.n};
+    if (CA.symm && coarseLocal) {
+        const auto k = coarseKernel(lev(l).nCoarse);
+        k.first<<<1, k.second, coarseLocalLds, c.stream>>>(a, csr, sk);
+    } else if (CA.symm)
         kCoarsePCG<<<1, 1024, coarseLds, c.stream>>>(a, sk);
     else
         kCoarseBiCG<<<1, 1024, coarseLds, c.stream>>>(a, sk);
