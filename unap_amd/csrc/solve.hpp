@@ -179,54 +179,63 @@ void runSchedule(SweepArgs<T, TV> a, const std::vector<int>& levStartH, int maxR
     }
 }
 
-// Sweeps by a group of workgroups on one XCD (sweep_group.hpp).  A level costs
-// the group about 0.9 us plus its share of the packed table at the 0.5 TB/s one
-// XCD draws; launched, it costs about 5 us plus the same at the whole chip's
-// rate (kSweepLevel / kGsLevelLanes), or 1-3 us in the one-workgroup tail.  The
-// lines below are where the two meet, in table bytes a level (MI355X): DIC
-// FP32 224k rows (0.68 MB) 115 against 155 us an application, DILU FP32 466k
-// rows (1.57 MB) 195 against 155; Gauss-Seidel FP64 on 105k rows of 17 entries
-// (1.3 MB) 3.4 against 5.5 us a level, on 220k of 15 (3.2 MB) 7.1 against 6.4.
-constexpr double kGroupLuBytes = 0.9e6, kGroupGsBytes = 1.6e6;
-constexpr int kGroupCUs = 32;  // workgroups a group on one XCD has when all its CUs are free
+// Sweeps by a group of workgroups (sweep_group.hpp) on one XCD, on all, or
+// launched level by level, by the packed table's bytes a level.  A level costs
+// a group on one XCD about 0.9 us plus the bytes at the 0.5 TB/s one XCD draws;
+// a group on all about 2 us (its barrier crosses XCDs) plus them at about 2.5
+// TB/s; a launch about 5 us plus the unpacked bytes at the whole chip's rate
+// with every wavefront slot filled.  The lines lie where they meet (MI355X):
+//   Gauss-Seidel, one sweep of a box, us (levels / one XCD / all):
+//     48^3 FP64 0.79 MB: - / 44 / 51      64^3 FP32 1.3 MB: - / 66 / 58
+//     100^3 FP64 6 MB: 102 / - / 84       128^3 FP64 12 MB: 145 / - / 145
+//     160^3 FP32 17 MB: 174 / - / 200
+//   DIC / DILU, a solve's iterations, ms:
+//     71x50x63 FP32 0.68 MB: 73 / 60 / 57      64^3 FP64 1.1 MB: 8.2 / - / 6.0
+//     128^3 FP64 7.6 MB: 18.7 / - / 17.3       160^3 FP64 14 MB: 29.1 / - / 30.3
+constexpr double kGroupLuOne = 0.6e6, kGroupLuAll = 9.0e6, kGroupGsOne = 1.0e6, kGroupGsAll = 12.0e6;
+constexpr int kGroupCUs = 32;  // workgroups an XCD has room for
 
-// The sweep schedules the packed tables serve: level-major order (position =
-// row), level bounds that fit the launch's LDS list.
+enum class GroupSpan { none, one, all };
+// The packed tables need the level-major order (position = row) and level
+// bounds that fit the launch's LDS list.
 template <typename T>
-bool groupSchedule(const DevMatrix<T>& M, size_t levels) {
-    return !M.fwdRows.p && levels <= (size_t)kGroupLevels;
+GroupSpan groupSpan(const DevMatrix<T>& M, size_t levels, double bytesALevel, double one, double all) {
+    if (M.fwdRows.p || levels > (size_t)kGroupLevels) return GroupSpan::none;
+    return bytesALevel <= one ? GroupSpan::one : (bytesALevel <= all ? GroupSpan::all : GroupSpan::none);
 }
 template <typename T>
-bool groupGsFits(const DevMatrix<T>& M) {
+GroupSpan groupGsSpan(const DevMatrix<T>& M) {
     const size_t nl = M.fwdStartH.size() - 1;
-    return groupSchedule(M, nl) && 16.0 * GroupPack<T>::kGs * M.gsLanes() * M.n <= kGroupGsBytes * (double)nl;
+    return groupSpan(M, nl, 16.0 * GroupPack<T>::kGs * M.gsLanes() * M.n / (double)nl, kGroupGsOne, kGroupGsAll);
 }
 template <typename T>
-bool groupLuFits(const DevMatrix<T>& M) {
+GroupSpan groupLuSpan(const DevMatrix<T>& M) {
     const size_t nl = M.fwdStartH.size() - 1;
-    return groupSchedule(M, nl + M.bwdStartH.size() - 1) &&
-           16.0 * GroupPack<T>::kLu * M.n <= kGroupLuBytes * (double)nl;
+    return groupSpan(M, nl + M.bwdStartH.size() - 1, 16.0 * GroupPack<T>::kLu * M.n / (double)nl, kGroupLuOne,
+                     kGroupLuAll);
 }
-inline GroupCtl groupCtl() {
+// kernel(args, control, skip) over every CU: a group on one XCD is the part of
+// the launch that lands there.
+template <class Kernel, class Args>
+void launchGroup(Kernel kernel, int threads, const Args& a, GroupSpan span, Skip sk) {
     Ctx& c = Ctx::get();
-    return {c.group.get(), const_cast<int*>(c.groupFail), kGroupCUs, 1};
+    const GroupCtl ctl{c.group.get(), const_cast<int*>(c.groupFail),
+                       span == GroupSpan::one ? kGroupCUs : kXcds * kGroupCUs};
+    kernel<<<kXcds * kGroupCUs, threads, 0, c.stream>>>(a, ctl, sk);
+    UH_LAUNCHED();
 }
 
 template <typename T>
-void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, Skip sk) {
-    Ctx& cx = Ctx::get();
-    const GroupTab& t = M.gsTable(cx.stream);
+void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, GroupSpan span, Skip sk) {
+    const GroupTab& t = M.gsTable(Ctx::get().stream);
     const GroupGs<T> g{t.tab.get(), t.ovf.get(), t.grp0.get(), M.fwdStart.get(), (int)M.fwdStartH.size() - 1, nSweeps,
                        x, b};
-    const GroupCtl c = groupCtl();
-    const int grid = 8 * c.expect, lpr = M.gsLanes();  // workgroups go to the eight XCDs in turn
-    if (lpr == 2)
-        kGroupGs<true, 2><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
-    else if (lpr == 4)
-        kGroupGs<true, 4><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
-    else
-        kGroupGs<true, 8><<<grid, kGsThreads, 0, cx.stream>>>(g, c, sk);
-    UH_LAUNCHED();
+    const bool one = span == GroupSpan::one;
+    switch (M.gsLanes()) {
+        case 2: launchGroup(one ? kGroupGs<true, 2, T> : kGroupGs<false, 2, T>, kGsThreads, g, span, sk); break;
+        case 4: launchGroup(one ? kGroupGs<true, 4, T> : kGroupGs<false, 4, T>, kGsThreads, g, span, sk); break;
+        default: launchGroup(one ? kGroupGs<true, 8, T> : kGroupGs<false, 8, T>, kGsThreads, g, span, sk);
+    }
 }
 
 // Gauss-Seidel smoothing, nSweeps forward sweeps (lduGaussSeidelSmoother.cpp:40-79).
@@ -234,8 +243,9 @@ template <typename T>
 void gsSmooth(DevMatrix<T>& M, T* x, const T* b, int nSweeps, Skip sk) {
     if (!M.sweepable) throw Error(-3, "Gauss-Seidel needs faces sorted by owner with owner < neighbour");
     SweepArgs<T, T> a{M.view(), x, b, nullptr, M.fwdRows.p, M.fwdStart.get()};
-    if (nSweeps > 0 && groupGsFits(M)) {
-        groupGs(M, x, b, nSweeps, sk);
+    const GroupSpan span = nSweeps > 0 ? groupGsSpan(M) : GroupSpan::none;
+    if (span != GroupSpan::none) {
+        groupGs(M, x, b, nSweeps, span, sk);
         return;
     }
     const int nl = (int)M.fwdStartH.size() - 1;
@@ -259,14 +269,13 @@ void luSweeps(DevMatrix<T>& M, bool dic, TV* w, const TV* r, const TV* rD, Skip 
     if constexpr (std::is_same<T, TV>::value) {
         // (DIC on asymmetric storage, with its second coefficient array, and
         // callers without the position-ordered rD run level by level)
-        if (groupLuFits(M) && !M.valU.p && rDpos) {
-            Ctx& cx = Ctx::get();
-            const GroupTab& t = M.luTable(cx.stream);
-            const GroupLu<T> g{Av, M.bwdView(cx.stream), t.tab.get(), t.grp0.get(), M.fwdStart.get(), M.bwdStart.get(),
+        const GroupSpan span = M.valU.p || !rDpos ? GroupSpan::none : groupLuSpan(M);
+        if (span != GroupSpan::none) {
+            hipStream_t s = Ctx::get().stream;
+            const GroupTab& t = M.luTable(s);
+            const GroupLu<T> g{Av, M.bwdView(s), t.tab.get(), t.grp0.get(), M.fwdStart.get(), M.bwdStart.get(),
                                (int)M.fwdStartH.size() - 1, (int)M.bwdStartH.size() - 1, r, rD, rDpos, w};
-            const GroupCtl c = groupCtl();
-            kGroupLu<true><<<8 * c.expect, kLuThreads, 0, cx.stream>>>(g, c, sk);
-            UH_LAUNCHED();
+            launchGroup(span == GroupSpan::one ? kGroupLu<true, T> : kGroupLu<false, T>, kLuThreads, g, span, sk);
             return;
         }
     }

@@ -6,51 +6,64 @@
 // tail has one CU's gather rate.  Here a group of resident workgroups walks
 // all levels (and all sweeps of a smoothing call) behind a barrier of its own.
 // On one XCD that barrier is a store and a poll in the L2 that its CUs share:
-// 0.2 us a hop, against 0.4 us across XCDs and 0.25 us for one returning
-// atomic (11 ns apart on one address, so counting arrivals or handing out
-// rows by atomics would cost more than the levels).
+// 0.2 us a hop and 0.3 us in all, against 0.4 us a hop across XCDs and 0.25 us
+// for one returning atomic (11 ns apart on one address, so counting arrivals
+// or handing out rows by atomics would cost more than the levels).
 //
 // Joining.  A launch holds more workgroups than take part.  Each one that
-// starts reads the XCD it runs on; the first to arrive elects its XCD (unless
-// the group spans all), and workgroups there register until the first
-// registrant closes the list: when all expected are in, or a few microseconds
-// later.  Only registered, and therefore running, workgroups take part, so no
-// barrier ever waits for a workgroup that has no place on the device, and the
-// work is split by the number that registered.  The rest leave at once.  The
-// last workgroup of the launch to leave clears the list for the next one.
+// starts reads the XCD it runs on and registers there (on one XCD: the first
+// to arrive elects its own, and the others leave); the first closes the list
+// when all expected are in, or a few microseconds later.  Only registered, and
+// therefore running, workgroups take part, so no barrier ever waits for a
+// workgroup that has no place on the device, and the work is split by the
+// number that registered.  A wait that never ends all the same (a fault in
+// this scheme) gives up after some seconds and is reported to the host.
 //
 // Visibility.  Values that cross workgroups (the swept vector, the flags) are
-// read with agent-scope loads, which pass the CU's own cache and are answered
-// by the L2, and stored through to it; a wavefront waits for its stores'
-// acknowledgement before its workgroup raises its flag.
+// read with agent-scope loads, which pass the CU's own cache; the group on one
+// XCD stores them to the L2 those loads are answered from, a wider group
+// through it (agent scope).  A wavefront waits for its stores' acknowledgement
+// before its workgroup raises its flag.
 #pragma once
 
 #include "ops.hpp"
 
 namespace unap_hip {
 
-constexpr int kGroupMax = 256;           // workgroups that may take part
+constexpr int kXcds = 8;
+constexpr int kGroupPerXcd = 32;         // workgroups of one XCD that may take part
 constexpr unsigned kGroupClosed = 1u << 31;
 constexpr int kGroupSpinLimit = 1 << 23; // polls before a wait gives up (seconds)
 
-// One word a 128-byte line, the flags packed 32 a line; all zero between launches.
+// Words written by different workgroups at different times lie on lines of
+// their own; words polled together share one.  The words of the list are zero
+// between launches.  The steps are never reset: they count on from launch to
+// launch (epoch), because an XCD's own flags stay dirty in its L2, and a reset
+// from another XCD would be undone when they are written back.
 struct GroupSync {
     unsigned elect[32];
-    unsigned reg[32];
-    unsigned parts[32];
     unsigned exits[32];
-    unsigned flag[kGroupMax];
+    unsigned reg[kXcds][32];             // registered workgroups
+    unsigned count[32];                  // 1 + the number that takes part, by XCD
+    unsigned epoch[32];                  // steps of all launches before
+    unsigned flag[kXcds][kGroupPerXcd];  // step reached, by workgroup
+    unsigned xflag[32];                  // step reached, by XCD
+    unsigned go[kXcds][32];              // step the XCD's workgroups may start
 };
 
 struct GroupCtl {
     GroupSync* s;
-    int* fail;    // host word: a wait gave up
-    int expect;   // workgroups the group is meant to have
-    int oneXcd;
+    int* fail;   // host word: a wait gave up
+    int expect;  // workgroups the group is meant to have
 };
 
+// A workgroup's place: ranks run through the XCDs in turn, so that neighbouring
+// ranks share an L2.  rank < 0: it takes no part.
 struct Group {
     int rank, size;
+    int xcd, local, localSize;
+    unsigned xcds;   // bit x: XCD x takes part
+    unsigned epoch;  // this launch's steps count from here
 };
 
 __device__ __forceinline__ unsigned groupPeek(const unsigned* p) {
@@ -69,61 +82,126 @@ __device__ __forceinline__ void gst(T* p, T v) {
         __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+template <bool One>
 __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
-    __shared__ int sRank, sSize;
-    if (threadIdx.x == 0) {
+    __shared__ Group sg;
+    if (threadIdx.x < 64) {  // the first wavefront, all lanes together
         GroupSync* S = c.s;
-        int rank = -1;
-        unsigned size = 0;
-        bool in = true;
-        if (c.oneXcd) {
-            const unsigned me = 1u + (__builtin_amdgcn_s_getreg((31 << 11) | 20) & 0xfu);  // HW_REG_XCC_ID
+        const int lane = (int)threadIdx.x;
+        const unsigned xcd = __builtin_amdgcn_s_getreg((31 << 11) | 20) & (kXcds - 1);  // HW_REG_XCC_ID
+        unsigned mine = kGroupClosed;
+        bool leader = false;
+        if (lane == 0) {
+            // one XCD: the first arrival's; all: the first arrival closes the list
             unsigned old = 0u;
+            const unsigned me = One ? 1u + xcd : 1u;
             __hip_atomic_compare_exchange_strong(&S->elect[0], &old, me, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
-            in = old == 0u || old == me;
+            if (!One || old == 0u || old == me)
+                mine = __hip_atomic_fetch_add(&S->reg[xcd][0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            leader = old == 0u;
         }
-        if (in) {
-            const unsigned r = __hip_atomic_fetch_add(&S->reg[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (!(r & kGroupClosed) && r < (unsigned)kGroupMax) {
-                rank = (int)r;
-                if (r == 0u) {
-                    const long long t0 = wall_clock64();  // 100 MHz
-                    while (groupPeek(&S->reg[0]) < (unsigned)c.expect && wall_clock64() - t0 < 400)
-                        __builtin_amdgcn_s_sleep(1);
-                    size = __hip_atomic_fetch_or(&S->reg[0], kGroupClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    size = size < (unsigned)kGroupMax ? size : (unsigned)kGroupMax;
-                    __hip_atomic_store(&S->parts[0], size, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                } else {
-                    int spins = 0;
-                    while ((size = groupPeek(&S->parts[0])) == 0u && ++spins < kGroupSpinLimit)
-                        __builtin_amdgcn_s_sleep(1);
-                    if (size == 0u) {
-                        *c.fail = 1;
-                        rank = -1;
-                    }
+        mine = __builtin_amdgcn_readfirstlane(mine);
+        leader = __builtin_amdgcn_readfirstlane((int)leader) != 0;
+        const bool in = !(mine & kGroupClosed) && mine < (unsigned)kGroupPerXcd;
+        unsigned count = 0u;  // lane x < 8: 1 + XCD x's workgroups
+        if (leader) {
+            const long long t0 = wall_clock64();  // 100 MHz
+            for (;;) {
+                unsigned r = lane < kXcds ? groupPeek(&S->reg[lane][0]) : 0u;
+#pragma unroll
+                for (int o = kXcds / 2; o >= 1; o >>= 1) r += __shfl_xor(r, o, 64);
+                if (__builtin_amdgcn_readfirstlane(r) >= (unsigned)c.expect || wall_clock64() - t0 >= 400) break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (lane < kXcds) {
+                const unsigned r = __hip_atomic_fetch_or(&S->reg[lane][0], kGroupClosed, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT);
+                count = 1u + (r < (unsigned)kGroupPerXcd ? r : (unsigned)kGroupPerXcd);
+                __hip_atomic_store(&S->count[lane], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else if (in) {
+            int spins = 0;
+            for (;;) {
+                count = lane < kXcds ? groupPeek(&S->count[lane]) : 1u;
+                if (!__any(count == 0u)) break;
+                if (++spins > kGroupSpinLimit) {
+                    *c.fail = 1;
+                    break;
                 }
+                __builtin_amdgcn_s_sleep(1);
             }
         }
-        sRank = rank;
-        sSize = (int)size;
+        Group g{-1, 0, (int)xcd, (int)mine, 0, 0u, 0u};
+        if (in) {
+            int before = 0;
+#pragma unroll
+            for (int x = 0; x < kXcds; ++x) {
+                const int k = (int)__builtin_amdgcn_readlane(count, x) - 1;
+                if (k < 0) continue;  // (a wait gave up)
+                if (x < (int)xcd) before += k;
+                if (x == (int)xcd) g.localSize = k;
+                g.size += k;
+                if (k > 0) g.xcds |= 1u << x;
+            }
+            if (g.local < g.localSize) g.rank = before + g.local;
+            g.epoch = groupPeek(&S->epoch[0]);  // changed by the launch's last workgroup only
+        }
+        if (lane == 0) sg = g;
     }
     __syncthreads();
-    return {sRank, sSize};
+    return sg;
 }
 
-// The end of a workgroup's part in the launch, participant or not.
-__device__ __forceinline__ void groupLeave(const GroupCtl& c) {
-    __shared__ int sLast;
+// The end of a workgroup's part in a launch of `steps` steps, participant or
+// not: the last workgroup of the launch clears the list and moves the epoch.
+__device__ __forceinline__ void groupLeave(const GroupCtl& c, unsigned steps) {
     __syncthreads();
-    if (threadIdx.x == 0)
-        sLast = __hip_atomic_fetch_add(&c.s->exits[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                gridDim.x - 1u;
-    __syncthreads();
-    if (!sLast) return;
-    unsigned* w = reinterpret_cast<unsigned*>(c.s);
-    for (unsigned i = threadIdx.x; i < sizeof(GroupSync) / sizeof(unsigned); i += blockDim.x)
-        __hip_atomic_store(w + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x != 0) return;
+    GroupSync* S = c.s;
+    if (__hip_atomic_fetch_add(&S->exits[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1u) return;
+    auto put = [](unsigned* p, unsigned v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    put(&S->epoch[0], groupPeek(&S->epoch[0]) + steps);
+    for (int x = 0; x < kXcds; ++x) {
+        put(&S->reg[x][0], 0u);
+        put(&S->count[x], 0u);
+    }
+    put(&S->elect[0], 0u);
+    put(&S->exits[0], 0u);
+}
+
+// Waits until the word this lane watches (null: none) is at least s, for every lane.
+__device__ __forceinline__ void groupAwait(const GroupCtl& c, const unsigned* p, unsigned s) {
+    int spins = 0;
+    for (;;) {
+        const unsigned f = p ? groupPeek(p) : s;
+        if (!__any((int)(f - s) < 0)) return;  // (the count may wrap)
+        if (++spins > kGroupSpinLimit) {
+            *c.fail = 1;
+            return;
+        }
+    }
+}
+// Step s of the group's barrier, by one wavefront of each workgroup.  Across
+// XCDs it goes by XCD: their first workgroups meet for the others, so that a
+// step's traffic between L2s is eight words rather than every flag to every L2.
+template <bool One>
+__device__ __forceinline__ void groupMeet(const GroupCtl& c, const Group& g, unsigned s) {
+    const int lane = (int)threadIdx.x & 63;
+    GroupSync* S = c.s;
+    if (lane == 0) gst<true>(&S->flag[g.xcd][g.local], s);
+    if constexpr (One) {
+        groupAwait(c, lane < g.localSize ? &S->flag[g.xcd][lane] : nullptr, s);
+        return;
+    }
+    if (g.local != 0) {
+        groupAwait(c, &S->go[g.xcd][0], s);
+        return;
+    }
+    groupAwait(c, lane < g.localSize ? &S->flag[g.xcd][lane] : nullptr, s);
+    if (lane == 0) gst<false>(&S->xflag[g.xcd], s);
+    groupAwait(c, lane < kXcds && (g.xcds >> lane & 1u) ? &S->xflag[lane] : nullptr, s);
+    if (lane == 0) gst<true>(&S->go[g.xcd][0], s);
 }
 
 // Roles of a workgroup's wavefronts.  The watcher raises the workgroup's flag
@@ -140,7 +218,7 @@ __device__ __forceinline__ void groupLeave(const GroupCtl& c) {
 // time, one such round being an item.  The group's barrier follows the last
 // item of a level, the workgroup's own follows every item.
 constexpr int kGroupLevels = 512;  // levels of a launch (bounds kept in LDS)
-constexpr int kRing = 3;
+constexpr int kRing = 2;
 
 struct GroupLevel {
     int first, count;  // this workgroup's groups in the table
@@ -211,28 +289,13 @@ struct GroupWalk {
 // The watcher's part.
 template <bool One>
 __device__ __forceinline__ void groupWatch(const GroupCtl& c, const Group& g, GroupWalk t) {
-    const int lane = (int)threadIdx.x & 63;
-    unsigned s = 0;
+    unsigned s = g.epoch;
     for (;;) {
         const bool last = t.lastOfLevel();
         t.next();
         if (t.done()) return;
         __builtin_amdgcn_s_barrier();
-        if (last) {
-            ++s;
-            if (lane == 0) gst<One>(&c.s->flag[g.rank], s);
-            for (int t0 = 0; t0 < g.size; t0 += 64) {
-                int spins = 0;
-                for (;;) {
-                    const unsigned f = t0 + lane < g.size ? groupPeek(&c.s->flag[t0 + lane]) : s;
-                    if (!__any(f < s)) break;
-                    if (++spins > kGroupSpinLimit) {
-                        *c.fail = 1;
-                        break;
-                    }
-                }
-            }
-        }
+        if (last) groupMeet<One>(c, g, ++s);
         __syncthreads();
     }
 }
@@ -441,7 +504,7 @@ __global__ void __launch_bounds__(kLuThreads) kGroupLu(GroupLu<T> a, GroupCtl c,
     __shared__ uint4 ring[kRing][NS][P][64];
     __shared__ GroupLevel lev[kGroupLevels];
     __shared__ int end[kGroupLevels];
-    const Group g = groupJoin(c);
+    const Group g = groupJoin<One>(c);
     if (g.rank >= 0) {
         const int nl = a.nFwd + a.nBwd;
         groupRuns<64, NS>(g, lev, end, a.fwdStart, a.grp0, a.nFwd);
@@ -547,7 +610,7 @@ __global__ void __launch_bounds__(kLuThreads) kGroupLu(GroupLu<T> a, GroupCtl c,
             groupLoad<NS, kLuLoaders, P>(a.tab, ring, t, wave - 1 - NS);
         }
     }
-    groupLeave(c);
+    groupLeave(c, (unsigned)(a.nFwd + a.nBwd));
 }
 
 // ------------------------------------------------------------ Gauss-Seidel
@@ -593,7 +656,7 @@ __global__ void __launch_bounds__(kGsThreads) kGroupGs(GroupGs<T> a, GroupCtl c,
     __shared__ T buf[NS * 64 * kGsS];
     __shared__ GroupLevel lev[kGroupLevels];
     __shared__ int end[kGroupLevels];
-    const Group g = groupJoin(c);
+    const Group g = groupJoin<One>(c);
     if (g.rank >= 0) {
         groupRuns<RW, NS>(g, lev, end, a.start, a.grp0, a.nl);
         __syncthreads();
@@ -682,7 +745,7 @@ __global__ void __launch_bounds__(kGsThreads) kGroupGs(GroupGs<T> a, GroupCtl c,
             groupLoad<NS, kGsLoaders, P>(a.tab, ring, t, wave - 1 - NS);
         }
     }
-    groupLeave(c);
+    groupLeave(c, (unsigned)(a.nl * a.nSweeps));
 }
 
 }  // namespace unap_hip
