@@ -536,15 +536,25 @@ struct FinEigAlpha {  // eigenDiagPCG.cpp:166-189
     __device__ void operator()(double (&t)[1]) const {
         st->alpha = st->rho / t[0];
         st->alphas[it] = st->alpha;
+        st->nIter = it + 1;
     }
 };
 
 // computeMaxEig (eigenDiagPCG.cpp:213-315): Lanczos tridiagonal from the CG
-// coefficients, Gershgorin range from [0,0], Sturm bisection to 1e-5.
+// coefficients, Gershgorin range from [0,0], Sturm bisection to 1e-5 or to
+// neighbouring doubles.  CG that met a zero residual early (FP32 levels with a
+// strong diagonal underflow within ten steps) has recorded st->nIter steps
+// only; without any, D^-1 A is taken as the identity.
 __device__ __forceinline__ void chebyTable(KState* st, double boost, double ratio);
 
-static __global__ void kLanczosMaxEig(KState* st, int m, double boost, double ratio) {
+static __global__ void kLanczosMaxEig(KState* st, int steps, double boost, double ratio) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    const int m = (int)min((long long)steps, st->nIter);
+    if (m <= 0) {
+        st->lambda = 1.0;
+        chebyTable(st, boost, ratio);
+        return;
+    }
     double dg[32], of[32];  // T[i][i], T[i][i+1]
     for (int i = 0; i < m; ++i) {
         dg[i] = (i == 0) ? 1.0 / st->alphas[i] : 1.0 / st->alphas[i] + st->betas[i] / st->alphas[i - 1];
@@ -562,10 +572,11 @@ static __global__ void kLanczosMaxEig(KState* st, int m, double boost, double ra
     double xn;
     do {
         xn = (lo + hi) * 0.5;
+        if (!(xn > lo && xn < hi)) break;
         int s = 0;
         double p0 = xn - dg[0];
         if (p0 < 0) s = 1;
-        double p1 = (xn - dg[1]) * p0 - of[0] * of[0];
+        double p1 = m > 1 ? (xn - dg[1]) * p0 - of[0] * of[0] : p0;
         if (p1 * p0 < 0) s++;
         for (int k = 2; k < m; ++k) {
             const double p2 = (xn - dg[k]) * p1 - of[k - 1] * of[k - 1] * p0;
