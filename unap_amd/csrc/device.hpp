@@ -248,6 +248,7 @@ struct DevMatrix {
     DBuf<int> bwdCol;
     DBuf<T> bwdVal;
     GroupTab gsTab, luTab;  // made on first use
+    DBuf<double> amulX;     // unap_hip_ldu_spmv's operand in this order, kept from call to call
 
     // Lanes a row of the Gauss-Seidel table: kGsS entries a lane cover the
     // average row and most of the spread.

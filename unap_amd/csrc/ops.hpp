@@ -46,6 +46,16 @@ struct BAmul {
     __device__ void operator()(int r) const { y[r] = rowAmul<T, T>(A, r, x); }
 };
 
+// y = A x with y in the caller's order: the rows' results go straight to their
+// places (no internal y to write and read back).
+struct BAmulOut {
+    DMat<double> A;
+    const double* x;
+    double* y;
+    const int* perm;
+    __device__ void operator()(int r) const { y[perm[r]] = rowAmul<double, double>(A, r, x); }
+};
+
 // r = b - A x (PCG.cpp:61-67), optional shadow copy r0 = r (PBiCGStab.cpp:76-79),
 // sum r*r for normFactor (unapMatrixSolver.cpp:12-16).
 template <typename T>
