@@ -7,6 +7,8 @@
 // the system's level schedule with workgroup barriers between levels.
 // Workgroups take systems from an atomic ticket in a largest-first order
 // (longest-processing-time scheduling), and exit when the queue is empty.
+// Where large systems would leave most CUs waiting for a few, teams of
+// workgroups on one XCD take them instead (kBatchTeams).
 // The block size, workgroups per CU and rows per wavefront pass are picked by
 // a small autotuner that times whole batch solves.
 #include "unap_hip.h"
@@ -50,6 +52,19 @@ struct SweepTab {
 };
 constexpr int kSweepPre = 4;  // entries a thread holds for its next row
 
+// Teams.  A large system's rows are more than one CU can gather for: a team of
+// workgroups on one XCD shares them (below, TeamComm).
+constexpr int kTeamMax = 8;
+struct alignas(256) TeamSlot {
+    // (number << 40 | workgroups << 32 | system) of the leader's last command;
+    // workgroups kTeamQuit: the queue is empty
+    unsigned long long command;
+    unsigned long long flag[kTeamMax];  // a workgroup's barrier count in that command
+    double sums[2][2][16];
+};
+constexpr unsigned kTeamQuit = 255;
+constexpr int kBatchXcds = 8;
+
 struct BatchArgs {
     const BatchSys* sys;
     const int* order;  // queue order (largest first)
@@ -73,6 +88,10 @@ struct BatchArgs {
     double relTol, tol;
     long long maxIter;
     unap_hip_perf* perf;
+    int team;             // workgroups a team holds (1: none)
+    unsigned* arrived;    // workgroups started on each XCD
+    TeamSlot* slots;      // slotsPerXcd an XCD
+    int slotsPerXcd;
 };
 
 __device__ __forceinline__ double bsum(double v, double* red) {
@@ -121,7 +140,16 @@ struct EllMat {
 };
 constexpr int kEllBatch = 8;
 
+// A value that another workgroup of the team stored: read from the L2, past
+// this CU's L1, which may hold an older line.
+template <bool Team, typename T>
+__device__ __forceinline__ T ldT(const T* p) {
+    if constexpr (Team) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return *p;
+}
+
 // rowAmul's arithmetic: acc = 0 + d x_i, then + v_k x[c_k] in entry order.
+template <bool Team = false>
 __device__ __forceinline__ double ellAmul(const EllMat& A, int i, const double* x) {
     const int len = (int)(A.info[i] & 0xffffu);
     double acc = 0.0 + A.diag[i] * x[i];
@@ -135,7 +163,7 @@ __device__ __forceinline__ double ellAmul(const EllMat& A, int i, const double* 
             v[j] = A.val[e];
         }
 #pragma unroll
-        for (int j = 0; j < kEllBatch; ++j) xv[j] = x[c[j]];
+        for (int j = 0; j < kEllBatch; ++j) xv[j] = ldT<Team>(x + c[j]);
 #pragma unroll
         for (int j = 0; j < kEllBatch; ++j)
             if (k0 + j < len) acc = acc + v[j] * xv[j];
@@ -173,15 +201,16 @@ __device__ __forceinline__ void loadSweepRow(SweepRow& R, const SweepTab& T, int
 
 // acc -= coef_j * w[col_j] in entry order (the DIC/DILU row arithmetic of
 // fwdRow / bwdRow: coef_j is the FP32 product rD * coefficient).
+template <bool Team = false>
 __device__ __forceinline__ float sweepRow(const SweepRow& R, const SweepTab& T, int p, float acc, const float* w) {
     float x[kSweepPre];
 #pragma unroll
     for (int j = 0; j < kSweepPre; ++j)
-        if (j < T.m) x[j] = w[R.c[j]];
+        if (j < T.m) x[j] = ldT<Team>(w + R.c[j]);
 #pragma unroll
     for (int j = 0; j < kSweepPre; ++j)
         if (j < R.cnt) acc = acc - R.v[j] * x[j];
-    for (int j = kSweepPre; j < R.cnt; ++j) acc = acc - T.coef[(size_t)j * T.n + p] * w[T.col[(size_t)j * T.n + p]];
+    for (int j = kSweepPre; j < R.cnt; ++j) acc = acc - T.coef[(size_t)j * T.n + p] * ldT<Team>(w + T.col[(size_t)j * T.n + p]);
     return acc;
 }
 
@@ -458,6 +487,332 @@ __device__ void batchBiCG(const BatchArgs& a, const SysView& s, int off, unap_hi
     }
 }
 
+// ---------------------------------------------------------------- teams
+// One workgroup gathers at one CU's rate: a sweep or an Amul touches a cache
+// line for nearly every entry, and a CU takes about one line a cycle (95k rows
+// under a random numbering: 555 us for the two sweeps, 285 us for the Amul of
+// an iteration, whatever the loop).  A team's workgroups sit on one XCD, so
+// what they store is in the L2 they share once the store has been acknowledged:
+// their barrier waits for that and exchanges flags, and what another workgroup
+// stored is read past the L1.  No cache is written back or invalidated (release
+// and acquire fences at device scope do both to the L2: 16 us a barrier).
+//
+// 96 systems of up to 110k rows: 371 -> 137 ms a solve; 512 systems: 491 -> 397.
+//
+// Rows are dealt out over the team.  Sums keep the single workgroup's order:
+// the terms are stored first, then virtual thread v adds rows v, v + BS, ... in
+// that order, the team holding its BS virtual threads between them, and the
+// wavefronts' sums are added in their order.  So every result is bitwise that
+// of one workgroup, whatever the team's size.
+//
+// A team's leader takes systems from the queue and posts them to the members
+// that have started; it never waits for a workgroup that may not be running.
+struct TeamComm {
+    TeamSlot* slot;
+    int rank, size;
+    unsigned long long step;  // number << 40 | barriers passed
+    int parity;
+
+    __device__ __forceinline__ void barrier() {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores are in the L2
+        __syncthreads();
+        ++step;
+        const int t = (int)threadIdx.x;
+        if (t < 64) {
+            if (t == 0) __hip_atomic_store(&slot->flag[rank], step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (t < size)
+                while (__hip_atomic_load(&slot->flag[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < step) {
+                }
+        }
+        __syncthreads();
+    }
+
+    // v[s] = sum over rows of f(i)[s], as bsum / bsum2 of one workgroup whose
+    // thread t adds rows t, t + BS, ...
+    template <int NS, class F>
+    __device__ __forceinline__ void sum(int n, double (&out)[NS], F&& f) {
+        constexpr int kAhead = 8;
+        const int nt = (int)blockDim.x, nw = nt >> 6, lane = (int)threadIdx.x & 63;
+        const int vw = ((int)threadIdx.x >> 6) * size + rank;  // virtual wavefront
+        if (vw < nw) {
+            double acc[NS];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) acc[s] = 0.0;
+            for (int i0 = vw * 64 + lane; i0 < n; i0 += kAhead * nt) {
+                double v[kAhead][NS];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) f(min(i0 + u * nt, n - 1), v[u]);
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u)
+                    if (i0 + u * nt < n) {
+#pragma unroll
+                        for (int s = 0; s < NS; ++s) acc[s] += v[u][s];
+                    }
+            }
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+#pragma unroll
+                for (int o = 32; o >= 1; o >>= 1) acc[s] += __shfl_xor(acc[s], o, 64);
+                if (lane == 0) slot->sums[parity][s][vw] = acc[s];
+            }
+        }
+        barrier();
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            double a = 0.0;
+            for (int w = 0; w < nw; ++w) a += ldT<true>(&slot->sums[parity][s][w]);
+            out[s] = a;
+        }
+        parity ^= 1;
+    }
+};
+
+template <bool Fwd>
+__device__ __forceinline__ void teamSweep(TeamComm& c, const SweepTab& T, const int* start, int nl, const double* r,
+                                          float* w) {
+    const int nt = (int)blockDim.x * c.size, t = (int)blockDim.x * c.rank + (int)threadIdx.x;
+    SweepRow R;
+    int p = start[0] + t;
+    if (nl > 0 && p < start[1]) loadSweepRow(R, T, p);
+    for (int k = 0; k < nl; ++k) {
+        const int e = start[k + 1];
+        for (; p < e; p += nt) {
+            w[R.q] = sweepRow<true>(R, T, p, Fwd ? R.rd * (float)ldT<true>(r + R.q) : ldT<true>(w + R.q), w);
+            if (p + nt < e) loadSweepRow(R, T, p + nt);
+        }
+        p = e + t;
+        if (k + 1 < nl && p < start[k + 2]) loadSweepRow(R, T, p);
+        c.barrier();
+    }
+}
+__device__ __forceinline__ void teamPrecond(TeamComm& c, const SysView& s, const double* r, float* w) {
+    teamSweep<true>(c, s.fwd, s.fs, s.nFwd, r, w);
+    teamSweep<false>(c, s.bwd, s.bs, s.nBwd, r, w);
+}
+
+// batchPCG by a team
+__device__ void teamPCG(TeamComm& c, const BatchArgs& a, const SysView& s, int off, unap_hip_perf* pf) {
+    const int n = s.n, t = (int)blockDim.x * c.rank + (int)threadIdx.x, nt = (int)blockDim.x * c.size;
+    double* x = a.x + off;
+    const double* b = a.b + off;
+    double* r = a.v + off;
+    double* p = a.v + a.total + off;
+    double* w = a.v + 2 * a.total + off;
+    float* w32 = a.w32 + off;
+    double one[1], two[2];
+    auto L = [](const auto* q) { return ldT<true>(q); };
+    auto rr = [&](int i, double (&v)[1]) {
+        const double ri = L(r + i);
+        v[0] = ri * ri;
+    };
+    for (int i = t; i < n; i += nt) {
+        r[i] = b[i] - ellAmul(s.A, i, x);
+        p[i] = 0.0;
+        w[i] = 0.0;
+    }
+    c.barrier();
+    c.sum(n, one, rr);
+    const double init = sqrt(one[0]) + kSmallD;
+    double fin = init, prev = init, rho = 1.0e37, pq = 1.0;
+    long long it = 0;
+    int conv = 0, sing = 0;
+    for (;;) {
+        teamPrecond(c, s, r, w32);
+        c.sum(n, two, [&](int i, double (&v)[2]) {
+            const double z = (double)L(w32 + i);
+            v[0] = z * L(r + i);
+            v[1] = z * L(w + i);
+        });
+        rho = two[0];
+        if (!(fabs(rho) > kSmallD)) {
+            sing = 1;
+            break;
+        }
+        const double beta = -two[1] / pq;
+        vecRows<2, V2>(t, n, nt, [&](int i) { return V2{(double)L(w32 + i), p[i]}; },
+                       [&](int i, const V2& v) { p[i] = (it == 0) ? v.a : v.a + beta * v.b; });
+        c.barrier();
+        for (int i = t; i < n; i += nt) w[i] = ellAmul<true>(s.A, i, p);
+        c.barrier();
+        c.sum(n, one, [&](int i, double (&v)[1]) { v[0] = L(w + i) * L(p + i); });
+        pq = one[0];
+        const double alpha = rho / pq;
+        vecRows<2, V4>(t, n, nt, [&](int i) { return V4{x[i], p[i], r[i], w[i]}; },
+                       [&](int i, const V4& v) {
+                           x[i] = v.a + alpha * v.b;
+                           r[i] = v.c - alpha * v.d;
+                       });
+        c.barrier();
+        prev = fin;
+        c.sum(n, one, rr);
+        fin = sqrt(one[0]) + kSmallD;
+        ++it;
+        if (!(it < a.maxIter)) break;
+        if (bconv(fin, init, a.tol, a.relTol)) {
+            conv = 1;
+            break;
+        }
+    }
+    if (t == 0) {
+        pf->initial_residual = init;
+        pf->final_residual = fin;
+        pf->previous_residual = prev;
+        pf->n_iterations = it;
+        pf->converged = conv;
+        pf->singular = sing;
+    }
+}
+
+// batchBiCG by a team
+__device__ void teamBiCG(TeamComm& c, const BatchArgs& a, const SysView& s, int off, unap_hip_perf* pf) {
+    const int n = s.n, t = (int)blockDim.x * c.rank + (int)threadIdx.x, nt = (int)blockDim.x * c.size;
+    const long long T = a.total;
+    double* x = a.x + off;
+    const double* b = a.b + off;
+    double* r = a.v + off;
+    double* r0 = a.v + T + off;
+    double* p = a.v + 2 * T + off;
+    double* Ay = a.v + 3 * T + off;
+    double* sv = a.v + 4 * T + off;
+    double* t_ = a.v + 5 * T + off;
+    double* y = a.v + 6 * T + off;
+    double* z = a.v + 7 * T + off;
+    float* w32 = a.w32 + off;
+    double one[1], two[2];
+    auto L = [](const auto* q) { return ldT<true>(q); };
+    auto rr = [&](int i, double (&v)[1]) {
+        const double ri = L(r + i);
+        v[0] = ri * ri;
+    };
+    for (int i = t; i < n; i += nt) {
+        const double ri = b[i] - ellAmul(s.A, i, x);
+        r[i] = ri;
+        r0[i] = ri;
+        p[i] = 0.0;
+        Ay[i] = 0.0;
+    }
+    c.barrier();
+    c.sum(n, one, rr);
+    const double init = sqrt(one[0]) + kSmallD;
+    double fin = init, prev = init, rho = 0, alpha = 0, omega = 0;
+    double r0norm = init;
+    long long it = 0;
+    int k = 0;
+    int conv = 0, sing = 0;
+    for (;;) {
+        const double rhoOld = rho;
+        c.sum(n, one, [&](int i, double (&v)[1]) { v[0] = L(r0 + i) * L(r + i); });
+        rho = one[0];
+        if (k > 0 && fabs(rho) < kBicgRestart * r0norm * fin) {  // (batchBiCG)
+            for (int i = t; i < n; i += nt) r0[i] = r[i];
+            c.sum(n, one, rr);
+            rho = one[0];
+            r0norm = sqrt(rho);
+            k = 0;
+        }
+        if (!(fabs(rho) > kSmallD)) {
+            sing = 1;
+            break;
+        }
+        const double beta = (rho / rhoOld) * (alpha / omega);
+        vecRows<2, V3>(t, n, nt, [&](int i) { return V3{r[i], p[i], Ay[i]}; },
+                       [&](int i, const V3& v) { p[i] = (k == 0) ? v.a : v.a + beta * (v.b - omega * v.c); });
+        c.barrier();
+        teamPrecond(c, s, p, w32);
+        vecRows<2, V1>(t, n, nt, [&](int i) { return V1{(double)L(w32 + i)}; }, [&](int i, const V1& v) { y[i] = v.a; });
+        c.barrier();
+        for (int i = t; i < n; i += nt) Ay[i] = ellAmul<true>(s.A, i, y);
+        c.barrier();
+        c.sum(n, one, [&](int i, double (&v)[1]) { v[0] = L(r0 + i) * L(Ay + i); });
+        alpha = rho / one[0];
+        vecRows<2, V2>(t, n, nt, [&](int i) { return V2{r[i], Ay[i]}; },
+                       [&](int i, const V2& v) { sv[i] = v.a - alpha * v.b; });
+        c.barrier();
+        c.sum(n, one, [&](int i, double (&v)[1]) {
+            const double si = L(sv + i);
+            v[0] = si * si;
+        });
+        fin = sqrt(one[0]) + kSmallD;
+        if (bconv(fin, init, a.tol, a.relTol)) {
+            for (int i = t; i < n; i += nt) x[i] += alpha * y[i];
+            ++it;
+            conv = 1;
+            break;
+        }
+        teamPrecond(c, s, sv, w32);
+        vecRows<2, V1>(t, n, nt, [&](int i) { return V1{(double)L(w32 + i)}; }, [&](int i, const V1& v) { z[i] = v.a; });
+        c.barrier();
+        for (int i = t; i < n; i += nt) t_[i] = ellAmul<true>(s.A, i, z);
+        c.barrier();
+        c.sum(n, two, [&](int i, double (&v)[2]) {
+            const double ti = L(t_ + i);
+            v[0] = ti * ti;
+            v[1] = ti * L(sv + i);
+        });
+        omega = two[1] / two[0];
+        vecRows<2, V5>(t, n, nt, [&](int i) { return V5{y[i], z[i], sv[i], t_[i], x[i]}; },
+                       [&](int i, const V5& v) {
+                           x[i] = v.e + (alpha * v.a + omega * v.b);
+                           r[i] = v.c - omega * v.d;
+                       });
+        c.barrier();
+        prev = fin;
+        c.sum(n, one, rr);
+        fin = sqrt(one[0]) + kSmallD;
+        ++it;
+        ++k;
+        if (!(it < a.maxIter)) break;
+        if (bconv(fin, init, a.tol, a.relTol)) {
+            conv = 1;
+            break;
+        }
+    }
+    if (t == 0) {
+        pf->initial_residual = init;
+        pf->final_residual = fin;
+        pf->previous_residual = prev;
+        pf->n_iterations = it;
+        pf->converged = conv;
+        pf->singular = sing;
+    }
+}
+
+__device__ __forceinline__ SysView viewOf(const BatchArgs& a, const BatchSys& d) {
+    SysView s;
+    s.n = d.n;
+    s.A = {a.ellCol + d.ellOff, a.ellVal + d.ellOff, a.rowInfo + d.cellOff, a.diag + d.cellOff, d.n, d.ellW};
+    SweepTab* tabs[2] = {&s.fwd, &s.bwd};
+    for (int dir = 0; dir < 2; ++dir)
+        *tabs[dir] = {a.tabRc[dir] + d.cellOff, a.tabRd[dir] + d.cellOff, a.tabCol[dir] + d.tabOff[dir],
+                      a.tabCoef[dir] + d.tabOff[dir], d.n, d.tabM[dir]};
+    s.fs = a.fwdStart + d.fwdOff;
+    s.bs = a.bwdStart + d.bwdOff;
+    s.nFwd = d.nFwd;
+    s.nBwd = d.nBwd;
+    return s;
+}
+
+// One system by this workgroup alone.
+template <int VR>
+__device__ __forceinline__ void solveAlone(const BatchArgs& a, int sys, double* red) {
+    const BatchSys d = a.sys[sys];
+    const SysView s = viewOf(a, d);
+    if (d.type == UNAP_HIP_SOLVER_PCG)
+        batchPCG<VR>(a, s, d.cellOff, a.perf + sys, red);
+    else
+        batchBiCG<VR>(a, s, d.cellOff, a.perf + sys, red);
+    __syncthreads();
+}
+__device__ __forceinline__ void solveInTeam(TeamComm& c, const BatchArgs& a, int sys) {
+    const BatchSys d = a.sys[sys];
+    const SysView s = viewOf(a, d);
+    if (d.type == UNAP_HIP_SOLVER_PCG)
+        teamPCG(c, a, s, d.cellOff, a.perf + sys);
+    else
+        teamBiCG(c, a, s, d.cellOff, a.perf + sys);
+    c.barrier();  // all have read the last sums
+}
+
 template <int BS, int VR>
 __global__ void __launch_bounds__(BS) kBatchSolve(BatchArgs a) {
     __shared__ double red[32];
@@ -468,28 +823,90 @@ __global__ void __launch_bounds__(BS) kBatchSolve(BatchArgs a) {
         const int q = ticket;
         __syncthreads();
         if (q >= a.nsys) return;  // the queue is empty: every workgroup ends here
-        const BatchSys d = a.sys[a.order[q]];
-        SysView s;
-        s.n = d.n;
-        s.A = {a.ellCol + d.ellOff, a.ellVal + d.ellOff, a.rowInfo + d.cellOff, a.diag + d.cellOff, d.n, d.ellW};
-        SweepTab* tabs[2] = {&s.fwd, &s.bwd};
-        for (int dir = 0; dir < 2; ++dir)
-            *tabs[dir] = {a.tabRc[dir] + d.cellOff, a.tabRd[dir] + d.cellOff, a.tabCol[dir] + d.tabOff[dir],
-                          a.tabCoef[dir] + d.tabOff[dir], d.n, d.tabM[dir]};
-        s.fs = a.fwdStart + d.fwdOff;
-        s.bs = a.bwdStart + d.bwdOff;
-        s.nFwd = d.nFwd;
-        s.nBwd = d.nBwd;
-        if (d.type == UNAP_HIP_SOLVER_PCG)
-            batchPCG<VR>(a, s, d.cellOff, a.perf + a.order[q], red);
-        else
-            batchBiCG<VR>(a, s, d.cellOff, a.perf + a.order[q], red);
-        __syncthreads();
+        solveAlone<VR>(a, a.order[q], red);
     }
 }
 
-__global__ void kResetTicket(unsigned* t) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *t = 0u;
+// Workgroups worth having on a system: a level's barrier costs a team about as
+// much as one workgroup takes for kTeamRows rows of it.
+constexpr int kTeamRows = 256;
+__device__ __forceinline__ int teamWant(const BatchSys& d, int most) {
+    const int rows = d.n / max(1, max(d.nFwd, d.nBwd));
+    return min(most, (rows + kTeamRows - 1) / kTeamRows);
+}
+
+template <int BS, int VR>
+__global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
+    __shared__ double red[32];
+    __shared__ int sh[3];  // system, workgroups, number of the command
+    const unsigned xcd = __builtin_amdgcn_s_getreg((31 << 11) | 20) & (kBatchXcds - 1);  // HW_REG_XCC_ID
+    if (threadIdx.x == 0)
+        sh[0] = (int)__hip_atomic_fetch_add(&a.arrived[xcd], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int place = sh[0], first = place / a.team * a.team, rank = place - first;
+    TeamSlot* slot = a.slots + (size_t)xcd * a.slotsPerXcd + place / a.team;
+    __syncthreads();
+    auto post = [&](unsigned number, unsigned size, int sys) {
+        __hip_atomic_store(&slot->command,
+                           (unsigned long long)number << 40 | (unsigned long long)size << 32 | (unsigned)sys,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    unsigned number = 0;  // of the last command seen
+    for (;;) {
+        if (threadIdx.x == 0) {
+            if (rank == 0) {
+                const int q = (int)atomicAdd(a.ticket, 1u);
+                int size = (int)kTeamQuit, sys = 0;
+                if (q < a.nsys) {
+                    sys = a.order[q];
+                    const int want = teamWant(a.sys[sys], a.team);
+                    size = 1;
+                    for (int k = 0; want > 1 && k < 64; ++k) {  // the members start at about this time
+                        const int here = (int)__hip_atomic_load(&a.arrived[xcd], __ATOMIC_RELAXED,
+                                                                __HIP_MEMORY_SCOPE_AGENT) -
+                                         first;
+                        size = min(want, here);
+                        if (size == want) break;
+                        __builtin_amdgcn_s_sleep(16);
+                    }
+                }
+                ++number;
+                if (size > 1) post(number, (unsigned)size, sys);
+                sh[0] = sys;
+                sh[1] = size;
+            } else {
+                unsigned long long c;
+                while ((unsigned)((c = __hip_atomic_load(&slot->command, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT)) >> 40) == number)
+                    __builtin_amdgcn_s_sleep(4);
+                number = (unsigned)(c >> 40);
+                sh[0] = (int)(unsigned)c;
+                sh[1] = (int)((c >> 32) & 255u);
+            }
+            sh[2] = (int)number;
+        }
+        __syncthreads();
+        const int sys = sh[0], size = sh[1];
+        number = (unsigned)sh[2];
+        __syncthreads();
+        if (size == (int)kTeamQuit) return;  // the queue is empty
+        if (size == 1) {
+            solveAlone<VR>(a, sys, red);  // (posted to nobody)
+        } else if (rank < size) {
+            TeamComm c{slot, rank, size, (unsigned long long)number << 40, 0};
+            solveInTeam(c, a, sys);
+        }
+    }
+}
+
+__global__ void kResetQueue(unsigned* ticket, unsigned* arrived, TeamSlot* slots, int nSlots) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) *ticket = 0u;
+    if (t < kBatchXcds) arrived[t] = 0u;
+    if (t < nSlots) {
+        slots[t].command = 0ull;
+        for (int k = 0; k < kTeamMax; ++k) slots[t].flag[k] = 0ull;
+    }
 }
 
 }  // namespace unap_hip
@@ -512,6 +929,8 @@ struct unap_hip_batch_s {
     DBuf<float> tabRd[2], tabCoef[2];
     DBuf<int> tabCol[2];
     DBuf<unap_hip_perf> perf;
+    DBuf<unsigned> arrived;
+    DBuf<TeamSlot> slots;
     int blockSize = 0, wgPerCU = 0;  // 0 = not tuned yet
     int rowsPerThread = 4;           // vector-loop rows a thread (64 x this rows a wavefront pass)
     double lastMs = 0;
@@ -544,6 +963,19 @@ void launchShape(const BatchArgs& a, int grid, int vr, hipStream_t st) {
     }
 }
 
+// Workgroups a team (launches of 1024 threads): none where no system's average
+// level fills a workgroup; then 8, or 4 where the systems outnumber half the
+// CUs and their leaders would be too few.  ms a solve alone / teams of 4 / of 8
+// (MI355X, random numberings): 96 systems of 8..48 a side 364 / 175 / 141; 24
+// of 10..40 155 / 85 / 61; 300 of 8..40 207 / 143 / 231; 64 of 8..24, levels of
+// up to 920 rows 20.2 / 21.7 / 21.3.  Teams of 16: 206, 67, 425.
+int teamSize(const unap_hip_batch_s& B) {
+    int rows = 0;
+    for (const BatchSys& d : B.sysH) rows = std::max(rows, d.n / std::max(1, std::max(d.nFwd, d.nBwd)));
+    if (rows < 1024) return 1;
+    return 2 * B.nsys <= B.cus ? 8 : 4;
+}
+
 void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIter, int bs, int wgPerCU, int vr) {
     Ctx& c = Ctx::get();
     BatchArgs a;
@@ -573,8 +1005,22 @@ void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIt
     a.maxIter = maxIter;
     a.perf = B.perf.get();
     const int grid = std::max(1, std::min(B.nsys, B.cus * wgPerCU));
-    kResetTicket<<<1, 1, 0, c.stream>>>(B.ticket.get());
+    a.team = bs == 1024 ? teamSize(B) : 1;
+    a.arrived = B.arrived.get();
+    a.slots = B.slots.get();
+    a.slotsPerXcd = B.cus;
+    const int nSlots = (int)B.slots.n;
+    kResetQueue<<<(nSlots + 255) / 256, 256, 0, c.stream>>>(B.ticket.get(), B.arrived.get(), B.slots.get(), nSlots);
     UH_LAUNCHED();
+    if (a.team > 1) {
+        switch (vr) {
+            case 1: kBatchTeams<1024, 1><<<B.cus, 1024, 0, c.stream>>>(a); break;
+            case 2: kBatchTeams<1024, 2><<<B.cus, 1024, 0, c.stream>>>(a); break;
+            default: kBatchTeams<1024, 4><<<B.cus, 1024, 0, c.stream>>>(a); break;
+        }
+        UH_LAUNCHED();
+        return;
+    }
     switch (bs) {
         case 256: launchShape<256>(a, grid, vr, c.stream); break;
         case 512: launchShape<512>(a, grid, vr, c.stream); break;
@@ -768,6 +1214,8 @@ int unap_hip_batch_create(int64_t nsys, const int64_t* cellOff, const int64_t* f
         hipDeviceProp_t p;
         UH_CHECK(hipGetDeviceProperties(&p, dev));
         B->cus = p.multiProcessorCount;
+        B->arrived.alloc(kBatchXcds);
+        B->slots.alloc((size_t)kBatchXcds * B->cus);
         *out = guardB.release();
     });
 }
