@@ -228,13 +228,17 @@ void launchGroup(Kernel kernel, int threads, const Args& a, GroupSpan span, Skip
 template <typename T>
 void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, GroupSpan span, Skip sk) {
     const GroupTab& t = M.gsTable(Ctx::get().stream);
-    const GroupGs<T> g{t.tab.get(), t.ovf.get(), t.grp0.get(), M.fwdStart.get(), (int)M.fwdStartH.size() - 1, nSweeps,
-                       x, b};
+    const int nl = (int)M.fwdStartH.size() - 1;
     const bool one = span == GroupSpan::one;
-    switch (M.gsLanes()) {
-        case 2: launchGroup(one ? kGroupGs<true, 2, T> : kGroupGs<false, 2, T>, kGsThreads, g, span, sk); break;
-        case 4: launchGroup(one ? kGroupGs<true, 4, T> : kGroupGs<false, 4, T>, kGsThreads, g, span, sk); break;
-        default: launchGroup(one ? kGroupGs<true, 8, T> : kGroupGs<false, 8, T>, kGsThreads, g, span, sk);
+    for (int left = nSweeps; left > 0;) {
+        const int k = groupSweeps(nl, left);
+        const GroupGs<T> g{t.tab.get(), t.ovf.get(), t.grp0.get(), M.fwdStart.get(), nl, k, x, b};
+        switch (M.gsLanes()) {
+            case 2: launchGroup(one ? kGroupGs<true, 2, T> : kGroupGs<false, 2, T>, kGsThreads, g, span, sk); break;
+            case 4: launchGroup(one ? kGroupGs<true, 4, T> : kGroupGs<false, 4, T>, kGsThreads, g, span, sk); break;
+            default: launchGroup(one ? kGroupGs<true, 8, T> : kGroupGs<false, 8, T>, kGsThreads, g, span, sk);
+        }
+        left -= k;
     }
 }
 

@@ -26,6 +26,7 @@
 // before its workgroup raises its flag.
 #pragma once
 
+#include "group_steps.hpp"
 #include "ops.hpp"
 
 namespace unap_hip {
@@ -40,15 +41,20 @@ constexpr int kGroupSpinLimit = 1 << 23; // polls before a wait gives up (second
 // between launches.  The steps are never reset: they count on from launch to
 // launch (epoch), because an XCD's own flags stay dirty in its L2, and a reset
 // from another XCD would be undone when they are written back.
+template <typename W>
+struct GroupWords {
+    W flag[kXcds][kGroupPerXcd];    // step reached, by workgroup
+    W xflag[32];                    // step reached, by XCD
+    W go[kXcds][128 / sizeof(W)];   // step the XCD's workgroups may start
+};
 struct GroupSync {
     unsigned elect[32];
     unsigned exits[32];
     unsigned reg[kXcds][32];             // registered workgroups
     unsigned count[32];                  // 1 + the number that takes part, by XCD
-    unsigned epoch[32];                  // steps of all launches before
-    unsigned flag[kXcds][kGroupPerXcd];  // step reached, by workgroup
-    unsigned xflag[32];                  // step reached, by XCD
-    unsigned go[kXcds][32];              // step the XCD's workgroups may start
+    GroupStep epoch[16];                 // steps of all launches before
+    GroupWords<GroupStep> first;         // for a launch's first step
+    GroupWords<unsigned> next;           // for its others (group_steps.hpp)
 };
 
 struct GroupCtl {
@@ -62,11 +68,12 @@ struct GroupCtl {
 struct Group {
     int rank, size;
     int xcd, local, localSize;
-    unsigned xcds;   // bit x: XCD x takes part
-    unsigned epoch;  // this launch's steps count from here
+    unsigned xcds;    // bit x: XCD x takes part
+    GroupStep epoch;  // this launch's steps count from here
 };
 
-__device__ __forceinline__ unsigned groupPeek(const unsigned* p) {
+template <typename T>
+__device__ __forceinline__ T groupPeek(const T* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <typename T>
@@ -132,7 +139,7 @@ __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
                 __builtin_amdgcn_s_sleep(1);
             }
         }
-        Group g{-1, 0, (int)xcd, (int)mine, 0, 0u, 0u};
+        Group g{-1, 0, (int)xcd, (int)mine, 0, 0u, 0};
         if (in) {
             int before = 0;
 #pragma unroll
@@ -155,12 +162,12 @@ __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
 
 // The end of a workgroup's part in a launch of `steps` steps, participant or
 // not: the last workgroup of the launch clears the list and moves the epoch.
-__device__ __forceinline__ void groupLeave(const GroupCtl& c, unsigned steps) {
+__device__ __forceinline__ void groupLeave(const GroupCtl& c, GroupStep steps) {
     __syncthreads();
     if (threadIdx.x != 0) return;
     GroupSync* S = c.s;
     if (__hip_atomic_fetch_add(&S->exits[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1u) return;
-    auto put = [](unsigned* p, unsigned v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto put = [](auto* p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     put(&S->epoch[0], groupPeek(&S->epoch[0]) + steps);
     for (int x = 0; x < kXcds; ++x) {
         put(&S->reg[x][0], 0u);
@@ -171,11 +178,11 @@ __device__ __forceinline__ void groupLeave(const GroupCtl& c, unsigned steps) {
 }
 
 // Waits until the word this lane watches (null: none) is at least s, for every lane.
-__device__ __forceinline__ void groupAwait(const GroupCtl& c, const unsigned* p, unsigned s) {
+template <typename W>
+__device__ __forceinline__ void groupAwait(const GroupCtl& c, const W* p, W s) {
     int spins = 0;
     for (;;) {
-        const unsigned f = p ? groupPeek(p) : s;
-        if (!__any((int)(f - s) < 0)) return;  // (the count may wrap)
+        if (!__any(!groupReached(p ? groupPeek(p) : s, s))) return;
         if (++spins > kGroupSpinLimit) {
             *c.fail = 1;
             return;
@@ -185,23 +192,22 @@ __device__ __forceinline__ void groupAwait(const GroupCtl& c, const unsigned* p,
 // Step s of the group's barrier, by one wavefront of each workgroup.  Across
 // XCDs it goes by XCD: their first workgroups meet for the others, so that a
 // step's traffic between L2s is eight words rather than every flag to every L2.
-template <bool One>
-__device__ __forceinline__ void groupMeet(const GroupCtl& c, const Group& g, unsigned s) {
+template <bool One, typename W>
+__device__ __forceinline__ void groupMeet(const GroupCtl& c, const Group& g, GroupWords<W>& w, W s) {
     const int lane = (int)threadIdx.x & 63;
-    GroupSync* S = c.s;
-    if (lane == 0) gst<true>(&S->flag[g.xcd][g.local], s);
+    if (lane == 0) gst<true>(&w.flag[g.xcd][g.local], s);
     if constexpr (One) {
-        groupAwait(c, lane < g.localSize ? &S->flag[g.xcd][lane] : nullptr, s);
+        groupAwait<W>(c, lane < g.localSize ? &w.flag[g.xcd][lane] : nullptr, s);
         return;
     }
     if (g.local != 0) {
-        groupAwait(c, &S->go[g.xcd][0], s);
+        groupAwait<W>(c, &w.go[g.xcd][0], s);
         return;
     }
-    groupAwait(c, lane < g.localSize ? &S->flag[g.xcd][lane] : nullptr, s);
-    if (lane == 0) gst<false>(&S->xflag[g.xcd], s);
-    groupAwait(c, lane < kXcds && (g.xcds >> lane & 1u) ? &S->xflag[lane] : nullptr, s);
-    if (lane == 0) gst<true>(&S->go[g.xcd][0], s);
+    groupAwait<W>(c, lane < g.localSize ? &w.flag[g.xcd][lane] : nullptr, s);
+    if (lane == 0) gst<false>(&w.xflag[g.xcd], s);
+    groupAwait<W>(c, lane < kXcds && (g.xcds >> lane & 1u) ? &w.xflag[lane] : nullptr, s);
+    if (lane == 0) gst<true>(&w.go[g.xcd][0], s);
 }
 
 // Roles of a workgroup's wavefronts.  The watcher raises the workgroup's flag
@@ -289,13 +295,29 @@ struct GroupWalk {
 // The watcher's part.
 template <bool One>
 __device__ __forceinline__ void groupWatch(const GroupCtl& c, const Group& g, GroupWalk t) {
-    unsigned s = g.epoch;
+    const unsigned e = (unsigned)g.epoch;
+    unsigned s = e;
+    if (((int)threadIdx.x & 63) == 0) {  // this workgroup's words of the later steps
+        GroupWords<unsigned>& w = c.s->next;
+        gst<true>(&w.flag[g.xcd][g.local], e);
+        if (g.local == 0) {
+            gst<false>(&w.xflag[g.xcd], e);
+            gst<true>(&w.go[g.xcd][0], e);
+        }
+    }
     for (;;) {
         const bool last = t.lastOfLevel();
         t.next();
         if (t.done()) return;
         __builtin_amdgcn_s_barrier();
-        if (last) groupMeet<One>(c, g, ++s);
+        if (last) {
+            if (s++ == e) {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // those words are there before the first step's
+                groupMeet<One>(c, g, c.s->first, g.epoch + 1);
+            } else {
+                groupMeet<One>(c, g, c.s->next, s);
+            }
+        }
         __syncthreads();
     }
 }
@@ -610,7 +632,7 @@ __global__ void __launch_bounds__(kLuThreads) kGroupLu(GroupLu<T> a, GroupCtl c,
             groupLoad<NS, kLuLoaders, P>(a.tab, ring, t, wave - 1 - NS);
         }
     }
-    groupLeave(c, (unsigned)(a.nFwd + a.nBwd));
+    groupLeave(c, (GroupStep)(a.nFwd + a.nBwd));
 }
 
 // ------------------------------------------------------------ Gauss-Seidel
@@ -745,7 +767,7 @@ __global__ void __launch_bounds__(kGsThreads) kGroupGs(GroupGs<T> a, GroupCtl c,
             groupLoad<NS, kGsLoaders, P>(a.tab, ring, t, wave - 1 - NS);
         }
     }
-    groupLeave(c, (unsigned)(a.nl * a.nSweeps));
+    groupLeave(c, (GroupStep)a.nl * (GroupStep)a.nSweeps);
 }
 
 }  // namespace unap_hip
