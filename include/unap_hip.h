@@ -53,6 +53,12 @@ const char* unap_hip_last_error(void);
 #define UNAP_HIP_REDUCE_REFERENCE 1
 int unap_hip_set_reduction_order(int order);
 
+/* Polls that a workgroup of a sweep or a batch's team waits for another before
+   the call ends in UNAP_HIP_ERR_INTERNAL: 0 to 2^23, the default (seconds).
+   Applies to kernels launched or captured from then on.  No reference
+   counterpart; a wait that long is a fault of the device or of the library. */
+int unap_hip_set_wait_limit(int64_t polls);
+
 /* Solver iterations from the second on replayed from a HIP graph of one
    iteration (1, default) or launched one kernel at a time (0).  No reference
    counterpart; the results are identical either way.  The environment

@@ -1,8 +1,8 @@
 """The comparisons behind the group sweeps' barrier (group_steps.hpp), on the
-host.  A launch's first step: a word that no launch has refreshed must not
-count as reached, however many steps other launches have made since.  Its
-other steps: words that lie within the launch compare right wherever the
-32-bit count wraps.  A smoothing call of any number of sweeps is split so that
+host.  The meeting before a launch's first step: a word that no launch has
+refreshed must not count as reached, however many steps other launches have
+made since.  Its steps: words that lie within the launch compare right wherever
+the 32-bit count wraps.  A smoothing call of any number of sweeps is split so that
 no launch has more steps than those comparisons hold for."""
 import os
 import subprocess
@@ -22,7 +22,7 @@ int main() {
     const U64 steps[] = {1, 2, 3, 511, 512, 65537, 1 << 20, 0x7ffffffe};
     int bad = 0;
     for (U64 e : epochs) {
-        const GroupStep s = e + 1;  // the first step of a launch that starts at e
+        const GroupStep s = e + 1;  // the meeting of a launch that starts at e
         bad += !groupReached(s, s) || !groupReached(s + 1, s) || groupReached((GroupStep)e, s);
         for (U64 w : stale) bad += w <= e && groupReached((GroupStep)w, s);
         for (U64 k : steps)

@@ -92,6 +92,9 @@ struct BatchArgs {
     unsigned* arrived;    // workgroups started on each XCD
     TeamSlot* slots;      // slotsPerXcd an XCD
     int slotsPerXcd;
+    GroupStep* failed;    // (top bit) a wait between a team's workgroups gave up in this launch
+    int* fail;            // the same for the host
+    int waitLimit;        // polls before one does
 };
 
 __device__ __forceinline__ double bsum(double v, double* red) {
@@ -507,11 +510,16 @@ __device__ void batchBiCG(const BatchArgs& a, const SysView& s, int off, unap_hi
 //
 // A team's leader takes systems from the queue and posts them to the members
 // that have started; it never waits for a workgroup that may not be running.
+// A barrier that never ends all the same (a fault in this scheme) gives up
+// after some seconds, and with it the launch: the workgroup leaves its solve,
+// the others see the failure in their barriers, leaders end their teams.
 struct TeamComm {
     TeamSlot* slot;
     int rank, size;
     unsigned long long step;  // number << 40 | barriers passed
     int parity;
+    Waits waits;
+    int* dead;  // in LDS: this workgroup has given up a barrier
 
     __device__ __forceinline__ void barrier() {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores are in the L2
@@ -520,12 +528,13 @@ struct TeamComm {
         const int t = (int)threadIdx.x;
         if (t < 64) {
             if (t == 0) __hip_atomic_store(&slot->flag[rank], step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (t < size)
-                while (__hip_atomic_load(&slot->flag[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < step) {
-                }
+            waits.until((unsigned)step, [&] { return !__any(groupPeek(&slot->flag[t < size ? t : rank]) < step); });
+            if (waits.over && t == 0) *dead = 1;
         }
         __syncthreads();
     }
+    // (written before a barrier's last __syncthreads only)
+    __device__ __forceinline__ bool broken() const { return *dead != 0; }
 
     // v[s] = sum over rows of f(i)[s], as bsum / bsum2 of one workgroup whose
     // thread t adds rows t, t + BS, ...
@@ -647,7 +656,7 @@ __device__ void teamPCG(TeamComm& c, const BatchArgs& a, const SysView& s, int o
         c.sum(n, one, rr);
         fin = sqrt(one[0]) + kSmallD;
         ++it;
-        if (!(it < a.maxIter)) break;
+        if (!(it < a.maxIter) || c.broken()) break;
         if (bconv(fin, init, a.tol, a.relTol)) {
             conv = 1;
             break;
@@ -761,7 +770,7 @@ __device__ void teamBiCG(TeamComm& c, const BatchArgs& a, const SysView& s, int 
         fin = sqrt(one[0]) + kSmallD;
         ++it;
         ++k;
-        if (!(it < a.maxIter)) break;
+        if (!(it < a.maxIter) || c.broken()) break;
         if (bconv(fin, init, a.tol, a.relTol)) {
             conv = 1;
             break;
@@ -839,9 +848,12 @@ template <int BS, int VR>
 __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
     __shared__ double red[32];
     __shared__ int sh[3];  // system, workgroups, number of the command
+    __shared__ int dead;   // (TeamComm)
     const unsigned xcd = __builtin_amdgcn_s_getreg((31 << 11) | 20) & (kBatchXcds - 1);  // HW_REG_XCC_ID
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
+        dead = 0;
         sh[0] = (int)__hip_atomic_fetch_add(&a.arrived[xcd], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __syncthreads();
     const int place = sh[0], first = place / a.team * a.team, rank = place - first;
     TeamSlot* slot = a.slots + (size_t)xcd * a.slotsPerXcd + place / a.team;
@@ -875,6 +887,8 @@ __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
                 sh[0] = sys;
                 sh[1] = size;
             } else {
+                // No bound: the leader runs, and comes here after solves of at
+                // most maxIter iterations whose barriers are bounded.
                 unsigned long long c;
                 while ((unsigned)((c = __hip_atomic_load(&slot->command, __ATOMIC_RELAXED,
                                                          __HIP_MEMORY_SCOPE_AGENT)) >> 40) == number)
@@ -893,15 +907,23 @@ __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
         if (size == 1) {
             solveAlone<VR>(a, sys, red);  // (posted to nobody)
         } else if (rank < size) {
-            TeamComm c{slot, rank, size, (unsigned long long)number << 40, 0};
+            TeamComm c{slot, rank, size, (unsigned long long)number << 40, 0, Waits(a.waitLimit, a.failed, a.fail),
+                       &dead};
             solveInTeam(c, a, sys);
+            if (c.broken()) {
+                if (rank == 0 && threadIdx.x == 0) post(number + 1, kTeamQuit, 0);
+                return;
+            }
         }
     }
 }
 
-__global__ void kResetQueue(unsigned* ticket, unsigned* arrived, TeamSlot* slots, int nSlots) {
+__global__ void kResetQueue(unsigned* ticket, unsigned* arrived, GroupStep* failed, TeamSlot* slots, int nSlots) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) *ticket = 0u;
+    if (t == 0) {
+        *ticket = 0u;
+        *failed = 0ull;
+    }
     if (t < kBatchXcds) arrived[t] = 0u;
     if (t < nSlots) {
         slots[t].command = 0ull;
@@ -930,6 +952,7 @@ struct unap_hip_batch_s {
     DBuf<int> tabCol[2];
     DBuf<unap_hip_perf> perf;
     DBuf<unsigned> arrived;
+    DBuf<GroupStep> failed;
     DBuf<TeamSlot> slots;
     int blockSize = 0, wgPerCU = 0;  // 0 = not tuned yet
     int rowsPerThread = 4;           // vector-loop rows a thread (64 x this rows a wavefront pass)
@@ -1009,8 +1032,12 @@ void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIt
     a.arrived = B.arrived.get();
     a.slots = B.slots.get();
     a.slotsPerXcd = B.cus;
+    a.failed = B.failed.get();
+    a.fail = const_cast<int*>(c.groupFail);
+    a.waitLimit = c.waitLimit;
     const int nSlots = (int)B.slots.n;
-    kResetQueue<<<(nSlots + 255) / 256, 256, 0, c.stream>>>(B.ticket.get(), B.arrived.get(), B.slots.get(), nSlots);
+    kResetQueue<<<(nSlots + 255) / 256, 256, 0, c.stream>>>(B.ticket.get(), B.arrived.get(), B.failed.get(),
+                                                            B.slots.get(), nSlots);
     UH_LAUNCHED();
     if (a.team > 1) {
         switch (vr) {
@@ -1215,6 +1242,7 @@ int unap_hip_batch_create(int64_t nsys, const int64_t* cellOff, const int64_t* f
         UH_CHECK(hipGetDeviceProperties(&p, dev));
         B->cus = p.multiProcessorCount;
         B->arrived.alloc(kBatchXcds);
+        B->failed.alloc(1);
         B->slots.alloc((size_t)kBatchXcds * B->cus);
         *out = guardB.release();
     });
@@ -1257,6 +1285,7 @@ int unap_hip_batch_solve(unap_hip_batch B, double* x, const double* b, int where
             launchBatch(*B, relTol, tol, maxIter, bsz, wg, vr);
             UH_CHECK(hipEventRecord(e1, c.stream));
             UH_CHECK(hipEventSynchronize(e1));
+            c.sync();  // (throws before a failed launch's time is used)
             float ms = 0;
             UH_CHECK(hipEventElapsedTime(&ms, e0, e1));
             return (double)ms;
@@ -1266,24 +1295,27 @@ int unap_hip_batch_solve(unap_hip_batch B, double* x, const double* b, int where
             // workgroups per CU at 4 rows a thread, then the rows a thread
             // (1, 2, 4: 64, 128, 256 rows a wavefront pass) at the best shape
             double best = 1e300;
-            B->rowsPerThread = 4;
+            int bestBs = 0, bestWg = 0, bestVr = 4;
             for (int bsz : {256, 512, 1024})
                 for (int wg : {1, 2, 4}) {
                     if (bsz * wg > 2048) continue;
                     const double ms = timed(bsz, wg, 4);
                     if (ms < best) {
                         best = ms;
-                        B->blockSize = bsz;
-                        B->wgPerCU = wg;
+                        bestBs = bsz;
+                        bestWg = wg;
                     }
                 }
             for (int vr : {1, 2}) {
-                const double ms = timed(B->blockSize, B->wgPerCU, vr);
+                const double ms = timed(bestBs, bestWg, vr);
                 if (ms < best) {
                     best = ms;
-                    B->rowsPerThread = vr;
+                    bestVr = vr;
                 }
             }
+            B->blockSize = bestBs;
+            B->wgPerCU = bestWg;
+            B->rowsPerThread = bestVr;
         }
         B->lastMs = timed(B->blockSize, B->wgPerCU, B->rowsPerThread);
         (void)hipEventDestroy(e0);

@@ -86,9 +86,10 @@ struct Ctx {
     DBuf<KState> scratchState;  // for standalone calls (eigen estimate, precond apply)
     static Ctx& get();
     DBuf<GroupSync> group;             // meeting place of the group sweeps (sweep_group.hpp)
-    volatile int* groupFail = nullptr;  // pinned host word: one of their waits gave up
+    volatile int* groupFail = nullptr;  // pinned host word: a wait between workgroups gave up
+    int waitLimit = kWaitLimit;         // polls such a wait takes at most
     static Ctx* peek();  // the context if it exists (creating it allocates)
-    void sync();
+    void sync();         // throws if a wait has given up since the last call
 };
 
 struct Launch {

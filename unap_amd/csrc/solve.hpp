@@ -220,7 +220,7 @@ template <class Kernel, class Args>
 void launchGroup(Kernel kernel, int threads, const Args& a, GroupSpan span, Skip sk) {
     Ctx& c = Ctx::get();
     const GroupCtl ctl{c.group.get(), const_cast<int*>(c.groupFail),
-                       span == GroupSpan::one ? kGroupCUs : kXcds * kGroupCUs};
+                       span == GroupSpan::one ? kGroupCUs : kXcds * kGroupCUs, c.waitLimit};
     kernel<<<kXcds * kGroupCUs, threads, 0, c.stream>>>(a, ctl, sk);
     UH_LAUNCHED();
 }

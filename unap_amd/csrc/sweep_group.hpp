@@ -17,7 +17,10 @@
 // therefore running, workgroups take part, so no barrier ever waits for a
 // workgroup that has no place on the device, and the work is split by the
 // number that registered.  A wait that never ends all the same (a fault in
-// this scheme) gives up after some seconds and is reported to the host.
+// this scheme) gives up after some seconds.  That is reported to the host, and
+// from then on nothing waits: the workgroup that gave up goes through its
+// remaining steps without, the others see the failure in their waits, and the
+// launches queued behind leave at once, until the host has reported the error.
 //
 // Visibility.  Values that cross workgroups (the swept vector, the flags) are
 // read with agent-scope loads, which pass the CU's own cache; the group on one
@@ -34,7 +37,8 @@ namespace unap_hip {
 constexpr int kXcds = 8;
 constexpr int kGroupPerXcd = 32;         // workgroups of one XCD that may take part
 constexpr unsigned kGroupClosed = 1u << 31;
-constexpr int kGroupSpinLimit = 1 << 23; // polls before a wait gives up (seconds)
+constexpr int kWaitLimit = 1 << 23;      // polls before a wait gives up (seconds)
+constexpr int kWaitLook = 1 << 14;       // polls between looks at the failure word (milliseconds)
 
 // Words written by different workgroups at different times lie on lines of
 // their own; words polled together share one.  The words of the list are zero
@@ -52,15 +56,16 @@ struct GroupSync {
     unsigned exits[32];
     unsigned reg[kXcds][32];             // registered workgroups
     unsigned count[32];                  // 1 + the number that takes part, by XCD
-    GroupStep epoch[16];                 // steps of all launches before
-    GroupWords<GroupStep> first;         // for a launch's first step
-    GroupWords<unsigned> next;           // for its others (group_steps.hpp)
+    GroupStep epoch[16];                 // steps of all launches before; top bit: a wait gave up
+    GroupWords<unsigned> next;           // for a launch's steps (group_steps.hpp)
+    GroupWords<GroupStep> first;         // for the meeting before them, or the first
 };
 
 struct GroupCtl {
     GroupSync* s;
     int* fail;   // host word: a wait gave up
     int expect;  // workgroups the group is meant to have
+    int limit;   // polls before a wait gives up
 };
 
 // A workgroup's place: ranks run through the XCDs in turn, so that neighbouring
@@ -89,6 +94,49 @@ __device__ __forceinline__ void gst(T* p, T v) {
         __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A workgroup's waits on others, by one wavefront (all lanes together).  What
+// lies between two polls and after the last is part of a step's chain: one
+// counter runs through all waits, and what decides about giving up stands
+// apart.  (With a count and a state a wait, the sweeps on all XCDs took 3%
+// longer; with four polls a turn of the loop, 6%.)
+struct Waits {
+    int limit;          // polls before a wait gives up
+    GroupStep* failed;  // device (top bit) and host words of that
+    int* fail;
+    int polls;          // until the next look
+    int left = 0;       // of the limit, for the wait at step `at`
+    unsigned at = ~0u;
+    bool over = false;  // a wait has given up
+    __device__ __forceinline__ Waits(int l, GroupStep* d, int* h)
+        : limit(l), failed(d), fail(h), polls(min(l, kWaitLook)) {}
+    // Until done(), or given up; s: the step waited for.
+    template <class Done>
+    __device__ __forceinline__ void until(unsigned s, Done&& done) {
+        while (!done()) {
+            if (__builtin_expect(--polls >= 0, 1)) continue;
+            look(s);
+            if (over) return;
+        }
+    }
+    __device__ void look(unsigned s) {
+        polls = 0;  // once it is over, a wait's first poll looks and returns
+        if (s != at) {
+            at = s;
+            left = limit;
+        }
+        left -= kWaitLook;
+        over = groupBroken(groupPeek(failed));
+        if (over) return;
+        if (left >= 0) {
+            polls = kWaitLook;
+            return;
+        }
+        over = true;
+        __hip_atomic_fetch_or(failed, kGroupBroken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *fail = 1;
+    }
+};
+
 template <bool One>
 __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
     __shared__ Group sg;
@@ -110,7 +158,7 @@ __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
         }
         mine = __builtin_amdgcn_readfirstlane(mine);
         leader = __builtin_amdgcn_readfirstlane((int)leader) != 0;
-        const bool in = !(mine & kGroupClosed) && mine < (unsigned)kGroupPerXcd;
+        bool in = !(mine & kGroupClosed) && mine < (unsigned)kGroupPerXcd;
         unsigned count = 0u;  // lane x < 8: 1 + XCD x's workgroups
         if (leader) {
             const long long t0 = wall_clock64();  // 100 MHz
@@ -128,16 +176,14 @@ __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
                 __hip_atomic_store(&S->count[lane], count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         } else if (in) {
-            int spins = 0;
-            for (;;) {
-                count = lane < kXcds ? groupPeek(&S->count[lane]) : 1u;
-                if (!__any(count == 0u)) break;
-                if (++spins > kGroupSpinLimit) {
-                    *c.fail = 1;
-                    break;
-                }
+            Waits w(c.limit, &S->epoch[0], c.fail);
+            w.until(0u, [&] {
+                count = groupPeek(&S->count[lane & (kXcds - 1)]);
+                if (!__any(count == 0u)) return true;
                 __builtin_amdgcn_s_sleep(1);
-            }
+                return false;
+            });
+            in = !w.over;
         }
         Group g{-1, 0, (int)xcd, (int)mine, 0, 0u, 0};
         if (in) {
@@ -145,14 +191,13 @@ __device__ __forceinline__ Group groupJoin(const GroupCtl& c) {
 #pragma unroll
             for (int x = 0; x < kXcds; ++x) {
                 const int k = (int)__builtin_amdgcn_readlane(count, x) - 1;
-                if (k < 0) continue;  // (a wait gave up)
                 if (x < (int)xcd) before += k;
                 if (x == (int)xcd) g.localSize = k;
                 g.size += k;
                 if (k > 0) g.xcds |= 1u << x;
             }
-            if (g.local < g.localSize) g.rank = before + g.local;
-            g.epoch = groupPeek(&S->epoch[0]);  // changed by the launch's last workgroup only
+            g.epoch = groupPeek(&S->epoch[0]);  // but for the top bit, changed by the launch's last workgroup only
+            if (g.local < g.localSize && !groupBroken(g.epoch)) g.rank = before + g.local;
         }
         if (lane == 0) sg = g;
     }
@@ -177,36 +222,31 @@ __device__ __forceinline__ void groupLeave(const GroupCtl& c, GroupStep steps) {
     put(&S->exits[0], 0u);
 }
 
-// Waits until the word this lane watches (null: none) is at least s, for every lane.
+// Waits until the word this lane watches is at least s, for every lane (lanes
+// with none to watch take the workgroup's or XCD's own).
 template <typename W>
-__device__ __forceinline__ void groupAwait(const GroupCtl& c, const W* p, W s) {
-    int spins = 0;
-    for (;;) {
-        if (!__any(!groupReached(p ? groupPeek(p) : s, s))) return;
-        if (++spins > kGroupSpinLimit) {
-            *c.fail = 1;
-            return;
-        }
-    }
+__device__ __forceinline__ void groupAwait(Waits& wait, const W* p, W s) {
+    wait.until((unsigned)s, [&] { return !__any(!groupReached(groupPeek(p), s)); });
 }
 // Step s of the group's barrier, by one wavefront of each workgroup.  Across
 // XCDs it goes by XCD: their first workgroups meet for the others, so that a
 // step's traffic between L2s is eight words rather than every flag to every L2.
 template <bool One, typename W>
-__device__ __forceinline__ void groupMeet(const GroupCtl& c, const Group& g, GroupWords<W>& w, W s) {
+__device__ __forceinline__ void groupMeet(Waits& wait, const Group& g, GroupWords<W>& w, W s) {
     const int lane = (int)threadIdx.x & 63;
     if (lane == 0) gst<true>(&w.flag[g.xcd][g.local], s);
+    const W* flag = &w.flag[g.xcd][lane < g.localSize ? lane : g.local];
     if constexpr (One) {
-        groupAwait<W>(c, lane < g.localSize ? &w.flag[g.xcd][lane] : nullptr, s);
+        groupAwait<W>(wait, flag, s);
         return;
     }
     if (g.local != 0) {
-        groupAwait<W>(c, &w.go[g.xcd][0], s);
+        groupAwait<W>(wait, &w.go[g.xcd][0], s);
         return;
     }
-    groupAwait<W>(c, lane < g.localSize ? &w.flag[g.xcd][lane] : nullptr, s);
+    groupAwait<W>(wait, flag, s);
     if (lane == 0) gst<false>(&w.xflag[g.xcd], s);
-    groupAwait<W>(c, lane < kXcds && (g.xcds >> lane & 1u) ? &w.xflag[lane] : nullptr, s);
+    groupAwait<W>(wait, &w.xflag[lane < kXcds && (g.xcds >> lane & 1u) ? lane : g.xcd], s);
     if (lane == 0) gst<true>(&w.go[g.xcd][0], s);
 }
 
@@ -292,31 +332,39 @@ struct GroupWalk {
     }
 };
 
-// The watcher's part.
+// Sets a workgroup's words of the launch's steps (by its first wavefront,
+// which then has other loads to wait for).
+__device__ __forceinline__ void groupWords(const GroupCtl& c, const Group& g) {
+    if (threadIdx.x != 0) return;
+    const unsigned e = (unsigned)g.epoch;
+    GroupWords<unsigned>& w = c.s->next;
+    gst<true>(&w.flag[g.xcd][g.local], e);
+    if (g.local != 0) return;
+    gst<false>(&w.xflag[g.xcd], e);
+    gst<true>(&w.go[g.xcd][0], e);
+}
+// The watcher's part.  On one XCD the group meets on the 64-bit words before
+// the first step, while the loaders fill the ring.  Across XCDs a meeting takes
+// longer than that (4 us more a launch), so it is the first step's own.
 template <bool One>
 __device__ __forceinline__ void groupWatch(const GroupCtl& c, const Group& g, GroupWalk t) {
-    const unsigned e = (unsigned)g.epoch;
-    unsigned s = e;
-    if (((int)threadIdx.x & 63) == 0) {  // this workgroup's words of the later steps
-        GroupWords<unsigned>& w = c.s->next;
-        gst<true>(&w.flag[g.xcd][g.local], e);
-        if (g.local == 0) {
-            gst<false>(&w.xflag[g.xcd], e);
-            gst<true>(&w.go[g.xcd][0], e);
-        }
-    }
+    Waits wait(c.limit, &c.s->epoch[0], c.fail);
+    unsigned s = (unsigned)g.epoch;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the words are set before the others know
+    if constexpr (One) groupMeet<One>(wait, g, c.s->first, g.epoch + 1);
+    __syncthreads();
+    __syncthreads();
     for (;;) {
         const bool last = t.lastOfLevel();
         t.next();
         if (t.done()) return;
         __builtin_amdgcn_s_barrier();
         if (last) {
-            if (s++ == e) {
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // those words are there before the first step's
-                groupMeet<One>(c, g, c.s->first, g.epoch + 1);
-            } else {
-                groupMeet<One>(c, g, c.s->next, s);
-            }
+            if (!One && s == (unsigned)g.epoch)
+                groupMeet<One>(wait, g, c.s->first, g.epoch + 1);
+            else
+                groupMeet<One>(wait, g, c.s->next, s + 1u);
+            ++s;
         }
         __syncthreads();
     }
@@ -529,14 +577,13 @@ __global__ void __launch_bounds__(kLuThreads) kGroupLu(GroupLu<T> a, GroupCtl c,
     const Group g = groupJoin<One>(c);
     if (g.rank >= 0) {
         const int nl = a.nFwd + a.nBwd;
+        groupWords(c, g);
         groupRuns<64, NS>(g, lev, end, a.fwdStart, a.grp0, a.nFwd);
         groupRuns<64, NS>(g, lev + a.nFwd, end + a.nFwd, a.bwdStart, a.grp0 + a.nFwd, a.nBwd);
         __syncthreads();
         const int wave = groupWave(), lane = (int)threadIdx.x & 63;
         GroupWalk t(lev, end, nl, 1);
         if (wave == 0) {
-            __syncthreads();
-            __syncthreads();
             groupWatch<One>(c, g, t);
         } else if (wave <= NS) {
             const int tw = wave - 1;
@@ -680,13 +727,12 @@ __global__ void __launch_bounds__(kGsThreads) kGroupGs(GroupGs<T> a, GroupCtl c,
     __shared__ int end[kGroupLevels];
     const Group g = groupJoin<One>(c);
     if (g.rank >= 0) {
+        groupWords(c, g);
         groupRuns<RW, NS>(g, lev, end, a.start, a.grp0, a.nl);
         __syncthreads();
         const int wave = groupWave(), lane = (int)threadIdx.x & 63;
         GroupWalk t(lev, end, a.nl, a.nSweeps);
         if (wave == 0) {
-            __syncthreads();
-            __syncthreads();
             groupWatch<One>(c, g, t);
         } else if (wave <= NS) {
             const int tw = wave - 1, i = lane % LPR, wr = lane / LPR;

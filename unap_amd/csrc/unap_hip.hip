@@ -44,8 +44,13 @@ void Ctx::sync() {
     UH_CHECK(hipStreamSynchronize(stream));
     if (*groupFail) {
         *groupFail = 0;
-        UH_CHECK(hipMemset(group.get(), 0, sizeof(GroupSync)));
-        throw Error(UNAP_HIP_ERR_INTERNAL, "a sweep's workgroups waited too long for one another");
+        // (every launch has left its list clean; the step words stay as they are)
+        GroupStep e = 0;
+        GroupStep* epoch = &group.get()->epoch[0];
+        UH_CHECK(hipMemcpy(&e, epoch, sizeof e, hipMemcpyDeviceToHost));
+        e &= ~kGroupBroken;
+        UH_CHECK(hipMemcpy(epoch, &e, sizeof e, hipMemcpyHostToDevice));
+        throw Error(UNAP_HIP_ERR_INTERNAL, "workgroups waited too long for one another");
     }
 }
 
@@ -1056,6 +1061,13 @@ int unap_hip_set_reduction_order(int order) {
     return guard([&] {
         need(order == UNAP_HIP_REDUCE_TREE || order == UNAP_HIP_REDUCE_REFERENCE, "unknown reduction order");
         Ctx::get().serialReductions = order;
+    });
+}
+
+int unap_hip_set_wait_limit(int64_t polls) {
+    return guard([&] {
+        need(polls >= 0 && polls <= kWaitLimit, "the wait limit is 0 to 2^23 polls");
+        Ctx::get().waitLimit = (int)polls;
     });
 }
 

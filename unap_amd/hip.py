@@ -54,6 +54,7 @@ SIGNATURES = {
     "unap_hip_device_info": (ctypes.c_int, [ctypes.c_char_p, _i64, _i64p]),
     "unap_hip_set_reduction_order": (ctypes.c_int, [ctypes.c_int]),
     "unap_hip_set_graph_replay": (ctypes.c_int, [ctypes.c_int]),
+    "unap_hip_set_wait_limit": (ctypes.c_int, [_i64]),
     "unap_hip_ldu_create": (ctypes.c_int, [_i64, _i64, _i64p, _i64p, _f64p, _f64p, _f64p, ctypes.POINTER(_vp)]),
     "unap_hip_ldu_destroy": (ctypes.c_int, [_vp]),
     "unap_hip_ldu_info": (ctypes.c_int, [_vp, _i64p, _i64p, _intp, _i64p, _i64p]),
@@ -164,6 +165,11 @@ REDUCE_TREE, REDUCE_REFERENCE = 0, 1
 def set_reduction_order(order):
     """REDUCE_TREE (fast, default) or REDUCE_REFERENCE (the reference's serial sums)."""
     _check(lib().unap_hip_set_reduction_order(order))
+
+
+def set_wait_limit(polls=1 << 23):
+    """Polls that workgroups wait for one another before a call ends in an error."""
+    _check(lib().unap_hip_set_wait_limit(polls))
 
 
 def set_graph_replay(on):
