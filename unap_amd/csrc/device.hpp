@@ -22,6 +22,11 @@ struct Error : std::runtime_error {
     Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// Device memory has run out (the call that finds it leaves no error behind).
+struct OutOfMemory : Error {
+    using Error::Error;
+};
+
 #define UH_CHECK(expr)                                                                       \
     do {                                                                                     \
         hipError_t e_ = (expr);                                                              \
@@ -59,8 +64,16 @@ struct DBuf {
     ~DBuf() { release(); }
     void alloc(size_t count) {
         release();
+        if (!count) return;
+        const hipError_t e = hipMalloc((void**)&p, sizeof(T) * count);
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();
+            const std::string what = std::string("hipMalloc: ") + hipGetErrorString(e);
+            if (e == hipErrorOutOfMemory) throw OutOfMemory(-2, what);
+            throw Error(-2, what);
+        }
         n = count;
-        if (count) UH_CHECK(hipMalloc((void**)&p, sizeof(T) * count));
     }
     void release() {
         if (p) (void)hipFree(p);
@@ -194,11 +207,14 @@ __global__ void kBuildBwdCopy(DMat<T> A, const int* __restrict__ bwdRows, const 
 
 // Packed table of the group sweeps (sweep_group.hpp): groups of a wavefront's
 // rows, level by level.  The groups are made once; the entries are refilled
-// from the matrix after its values change, into the same buffers.
+// from the matrix after its values change, into the same buffers.  (A table
+// takes 160 bytes a row and more.  Where device memory does not hold it, the
+// matrix does without for good: its sweeps are launched level by level.)
 struct GroupTab {
     int rows = 0;  // rows a group
     int ng = 0;
     bool filled = false;
+    bool refused = false;
     DBuf<int2> grp;    // first schedule position and row count of a group
     DBuf<int> grp0;    // groups before each level
     DBuf<int> grpOvf;  // a group's first chunk in the overflow table
@@ -254,9 +270,27 @@ struct DevMatrix {
     // Lanes a row of the Gauss-Seidel table: kGsS entries a lane cover the
     // average row and most of the spread.
     int gsLanes() const { return entriesPerRow <= 7.0 ? 2 : (entriesPerRow <= 12.5 ? 4 : 8); }
-    // The tables need the level-major order (position = row).
-    const GroupTab& gsTable(hipStream_t s) {
-        GroupTab& t = gsTab;
+    // The tables need the level-major order (position = row).  Null: refused.
+    const GroupTab* gsTable(hipStream_t s) {
+        return whole(gsTab, [&](GroupTab& t) { makeGsTable(t, s); });
+    }
+    const GroupTab* luTable(hipStream_t s) {
+        return whole(luTab, [&](GroupTab& t) { makeLuTable(t, s); });
+    }
+    // A table whose making ran out of memory leaves none of its buffers.
+    template <class Make>
+    static const GroupTab* whole(GroupTab& t, Make&& make) {
+        if (t.refused) return nullptr;
+        try {
+            make(t);
+        } catch (const OutOfMemory&) {
+            t = GroupTab();
+            t.refused = true;
+            return nullptr;
+        }
+        return &t;
+    }
+    void makeGsTable(GroupTab& t, hipStream_t s) {
         const int lpr = gsLanes();
         if (!t.tab.p) {
             std::vector<int2> g;
@@ -275,8 +309,8 @@ struct DevMatrix {
             }
             t.grpOvf.upload(at, s);
             UH_CHECK(hipStreamSynchronize(s));
-            t.tab.alloc((size_t)t.ng * GroupPack<T>::kGs * 64);
             t.ovf.alloc((size_t)std::max(next, 1) * GroupPack<T>::kOvf * 64);
+            t.tab.alloc((size_t)t.ng * GroupPack<T>::kGs * 64);
             t.filled = false;
         }
         if (!t.filled) {
@@ -293,10 +327,8 @@ struct DevMatrix {
             UH_LAUNCHED();
             t.filled = true;
         }
-        return t;
     }
-    const GroupTab& luTable(hipStream_t s) {
-        GroupTab& t = luTab;
+    void makeLuTable(GroupTab& t, hipStream_t s) {
         if (!t.tab.p) {
             std::vector<int2> g;
             t.plan(fwdStartH, &bwdStartH, 64, g, s);
@@ -314,7 +346,6 @@ struct DevMatrix {
             UH_LAUNCHED();
             t.filled = true;
         }
-        return t;
     }
 
     DMat<T> view() const { return {n, sliceStart.get(), rowInfo.get(), col.get(), val.get(), diag.get()}; }
@@ -326,7 +357,7 @@ struct DevMatrix {
     // are the upper ones in both val and valU.
     DMat<T> bwdView(hipStream_t s) {
         if (!bwdVal.p) {
-            if (!bwdSlice.p) {
+            if (!bwdInfo.p) {
                 bwdSlice.upload(bwdSliceH, s);
                 bwdInfo.upload(bwdInfoH, s);
             }

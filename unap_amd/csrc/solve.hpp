@@ -226,13 +226,14 @@ void launchGroup(Kernel kernel, int threads, const Args& a, GroupSpan span, Skip
 }
 
 template <typename T>
-void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, GroupSpan span, Skip sk) {
-    const GroupTab& t = M.gsTable(Ctx::get().stream);
+bool groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, GroupSpan span, Skip sk) {
+    const GroupTab* t = M.gsTable(Ctx::get().stream);
+    if (!t) return false;
     const int nl = (int)M.fwdStartH.size() - 1;
     const bool one = span == GroupSpan::one;
     for (int left = nSweeps; left > 0;) {
         const int k = groupSweeps(nl, left);
-        const GroupGs<T> g{t.tab.get(), t.ovf.get(), t.grp0.get(), M.fwdStart.get(), nl, k, x, b};
+        const GroupGs<T> g{t->tab.get(), t->ovf.get(), t->grp0.get(), M.fwdStart.get(), nl, k, x, b};
         switch (M.gsLanes()) {
             case 2: launchGroup(one ? kGroupGs<true, 2, T> : kGroupGs<false, 2, T>, kGsThreads, g, span, sk); break;
             case 4: launchGroup(one ? kGroupGs<true, 4, T> : kGroupGs<false, 4, T>, kGsThreads, g, span, sk); break;
@@ -240,6 +241,7 @@ void groupGs(DevMatrix<T>& M, T* x, const T* b, int nSweeps, GroupSpan span, Ski
         }
         left -= k;
     }
+    return true;
 }
 
 // Gauss-Seidel smoothing, nSweeps forward sweeps (lduGaussSeidelSmoother.cpp:40-79).
@@ -248,10 +250,7 @@ void gsSmooth(DevMatrix<T>& M, T* x, const T* b, int nSweeps, Skip sk) {
     if (!M.sweepable) throw Error(-3, "Gauss-Seidel needs faces sorted by owner with owner < neighbour");
     SweepArgs<T, T> a{M.view(), x, b, nullptr, M.fwdRows.p, M.fwdStart.get()};
     const GroupSpan span = nSweeps > 0 ? groupGsSpan(M) : GroupSpan::none;
-    if (span != GroupSpan::none) {
-        groupGs(M, x, b, nSweeps, span, sk);
-        return;
-    }
+    if (span != GroupSpan::none && groupGs(M, x, b, nSweeps, span, sk)) return;
     const int nl = (int)M.fwdStartH.size() - 1;
     const int maxRows = tailRows(M.entriesPerRow);  // a GS row reads all its entries
     if (tailStart(M.fwdStartH, maxRows) == 0) {
@@ -274,10 +273,9 @@ void luSweeps(DevMatrix<T>& M, bool dic, TV* w, const TV* r, const TV* rD, Skip 
         // (DIC on asymmetric storage, with its second coefficient array, and
         // callers without the position-ordered rD run level by level)
         const GroupSpan span = M.valU.p || !rDpos ? GroupSpan::none : groupLuSpan(M);
-        if (span != GroupSpan::none) {
-            hipStream_t s = Ctx::get().stream;
-            const GroupTab& t = M.luTable(s);
-            const GroupLu<T> g{Av, M.bwdView(s), t.tab.get(), t.grp0.get(), M.fwdStart.get(), M.bwdStart.get(),
+        hipStream_t s = Ctx::get().stream;
+        if (const GroupTab* t = span != GroupSpan::none ? M.luTable(s) : nullptr) {
+            const GroupLu<T> g{Av, M.bwdView(s), t->tab.get(), t->grp0.get(), M.fwdStart.get(), M.bwdStart.get(),
                                (int)M.fwdStartH.size() - 1, (int)M.bwdStartH.size() - 1, r, rD, rDpos, w};
             launchGroup(span == GroupSpan::one ? kGroupLu<true, T> : kGroupLu<false, T>, kLuThreads, g, span, sk);
             return;
