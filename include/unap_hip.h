@@ -374,8 +374,8 @@ int unap_hip_ldu_renumber(int64_t n, int64_t n_faces, const int64_t* lower_addr,
 
 /* ------------------------------------------------------------------ batches
  * Many independent LDU systems solved in one persistent kernel launch: one
- * workgroup runs one system's whole Krylov solve, systems are taken from a
- * work queue largest-first.  System s has cells [cell_off[s], cell_off[s+1])
+ * workgroup, or a team of them, runs one system's whole Krylov solve, systems
+ * are taken from work queues largest-first.  System s has cells [cell_off[s], cell_off[s+1])
  * and faces [face_off[s], face_off[s+1]) of the concatenated arrays, with
  * addresses local to the system and faces owner-sorted.  solver[s] is
  * UNAP_HIP_SOLVER_PCG (with DIC) or UNAP_HIP_SOLVER_PBICGSTAB (with DILU);
@@ -400,6 +400,12 @@ int unap_hip_batch_config(unap_hip_batch B, int64_t* block_size, int64_t* wg_per
    128 or 256 (results do not depend on it). */
 int unap_hip_batch_set_config(unap_hip_batch B, int64_t block_size, int64_t wg_per_cu,
                               int64_t rows_per_wavefront);
+/* Workgroups on one XCD that share a large system, in launches of 1024
+   threads: 1 to 8 (1: none do), or 0 (default): chosen from the systems.
+   Results do not depend on it.  unap_hip_batch_team: the size in use since the
+   last solve (1: no teams) and the number of systems that teams take. */
+int unap_hip_batch_set_team(unap_hip_batch B, int64_t workgroups);
+int unap_hip_batch_team(unap_hip_batch B, int64_t* workgroups, int64_t* systems);
 
 #ifdef __cplusplus
 }

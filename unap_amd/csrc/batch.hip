@@ -8,7 +8,7 @@
 // Workgroups take systems from an atomic ticket in a largest-first order
 // (longest-processing-time scheduling), and exit when the queue is empty.
 // Where large systems would leave most CUs waiting for a few, teams of
-// workgroups on one XCD take them instead (kBatchTeams).
+// workgroups on one XCD take those (kBatchTeams, batch_plan.hpp).
 // The block size, workgroups per CU and rows per wavefront pass are picked by
 // a small autotuner that times whole batch solves.
 #include "unap_hip.h"
@@ -22,6 +22,7 @@
 #include <string>
 #include <vector>
 
+#include "batch_plan.hpp"
 #include "device.hpp"
 #include "ops.hpp"
 
@@ -54,22 +55,23 @@ constexpr int kSweepPre = 4;  // entries a thread holds for its next row
 
 // Teams.  A large system's rows are more than one CU can gather for: a team of
 // workgroups on one XCD shares them (below, TeamComm).
-constexpr int kTeamMax = 8;
 struct alignas(256) TeamSlot {
     // (number << 40 | workgroups << 32 | system) of the leader's last command;
-    // workgroups kTeamQuit: the queue is empty
+    // workgroups kTeamSolo: the team is over, each goes on by itself;
+    // kTeamQuit: the launch is broken
     unsigned long long command;
     unsigned long long flag[kTeamMax];  // a workgroup's barrier count in that command
     double sums[2][2][16];
 };
-constexpr unsigned kTeamQuit = 255;
+constexpr int kTeamLimit = 1 << 20;  // polls before a barrier gives up (tenths of a second)
+constexpr unsigned kTeamQuit = 255, kTeamSolo = 254;
 constexpr int kBatchXcds = 8;
 
 struct BatchArgs {
     const BatchSys* sys;
-    const int* order;  // queue order (largest first)
-    int nsys;
-    unsigned* ticket;
+    const int* order;  // queue order: nWide systems for teams, then the others, each largest first
+    int nsys, nWide;
+    unsigned* ticket;  // of the others, of the teams' systems, of the teams
     const uint32_t* rowInfo;
     const int* ellCol;
     const double* ellVal;
@@ -88,13 +90,13 @@ struct BatchArgs {
     double relTol, tol;
     long long maxIter;
     unap_hip_perf* perf;
-    int team;             // workgroups a team holds (1: none)
+    int team, teams;      // workgroups a team holds (1: none), teams at most
     unsigned* arrived;    // workgroups started on each XCD
     TeamSlot* slots;      // slotsPerXcd an XCD
     int slotsPerXcd;
     GroupStep* failed;    // (top bit) a wait between a team's workgroups gave up in this launch
     int* fail;            // the same for the host
-    int waitLimit;        // polls before one does
+    int waitLimit;        // polls before one does (an iteration has some 80 barriers)
 };
 
 __device__ __forceinline__ double bsum(double v, double* red) {
@@ -500,7 +502,7 @@ __device__ void batchBiCG(const BatchArgs& a, const SysView& s, int off, unap_hi
 // stored is read past the L1.  No cache is written back or invalidated (release
 // and acquire fences at device scope do both to the L2: 16 us a barrier).
 //
-// 96 systems of up to 110k rows: 371 -> 137 ms a solve; 512 systems: 491 -> 397.
+// 96 systems of up to 110k rows: 371 -> 131 ms a solve; 512 systems: 491 -> 302.
 //
 // Rows are dealt out over the team.  Sums keep the single workgroup's order:
 // the terms are stored first, then virtual thread v adds rows v, v + BS, ... in
@@ -511,14 +513,17 @@ __device__ void batchBiCG(const BatchArgs& a, const SysView& s, int off, unap_hi
 // A team's leader takes systems from the queue and posts them to the members
 // that have started; it never waits for a workgroup that may not be running.
 // A barrier that never ends all the same (a fault in this scheme) gives up
-// after some seconds, and with it the launch: the workgroup leaves its solve,
-// the others see the failure in their barriers, leaders end their teams.
+// after some tenths of a second.  The workgroup leaves its solve at the end of
+// the iteration, its team's others give up as well, a leader ends its team and
+// the workgroups on their own take no more systems.  (A barrier does no more
+// than count: the solve has no registers to spare, and looking at the others'
+// failure in the loop cost 96 systems 2 to 9%.)
 struct TeamComm {
     TeamSlot* slot;
     int rank, size;
     unsigned long long step;  // number << 40 | barriers passed
     int parity;
-    Waits waits;
+    const BatchArgs& a;
     int* dead;  // in LDS: this workgroup has given up a barrier
 
     __device__ __forceinline__ void barrier() {
@@ -528,8 +533,14 @@ struct TeamComm {
         const int t = (int)threadIdx.x;
         if (t < 64) {
             if (t == 0) __hip_atomic_store(&slot->flag[rank], step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            waits.until((unsigned)step, [&] { return !__any(groupPeek(&slot->flag[t < size ? t : rank]) < step); });
-            if (waits.over && t == 0) *dead = 1;
+            if (t < size) {
+                int polls = 0;
+                while (__hip_atomic_load(&slot->flag[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < step)
+                    if (++polls > a.waitLimit) {
+                        *dead = 1;
+                        break;
+                    }
+            }
         }
         __syncthreads();
     }
@@ -836,12 +847,9 @@ __global__ void __launch_bounds__(BS) kBatchSolve(BatchArgs a) {
     }
 }
 
-// Workgroups worth having on a system: a level's barrier costs a team about as
-// much as one workgroup takes for kTeamRows rows of it.
-constexpr int kTeamRows = 256;
-__device__ __forceinline__ int teamWant(const BatchSys& d, int most) {
-    const int rows = d.n / max(1, max(d.nFwd, d.nBwd));
-    return min(most, (rows + kTeamRows - 1) / kTeamRows);
+__host__ __device__ __forceinline__ int levelRows(const BatchSys& d) {
+    const int levels = d.nFwd > d.nBwd ? d.nFwd : d.nBwd;
+    return d.n / (levels > 1 ? levels : 1);
 }
 
 template <int BS, int VR>
@@ -863,15 +871,24 @@ __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
                            (unsigned long long)number << 40 | (unsigned long long)size << 32 | (unsigned)sys,
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
+    // The first a.teams leaders to start keep their teams until the teams'
+    // systems are taken; all other workgroups take the other systems alone.
+    const bool keep = rank == 0 && threadIdx.x == 0 && (int)atomicAdd(a.ticket + 2, 1u) < a.teams;
     unsigned number = 0;  // of the last command seen
+    bool solo = false;
     for (;;) {
         if (threadIdx.x == 0) {
-            if (rank == 0) {
+            if (solo) {
                 const int q = (int)atomicAdd(a.ticket, 1u);
-                int size = (int)kTeamQuit, sys = 0;
-                if (q < a.nsys) {
+                const bool take = q < a.nsys && !groupBroken(groupPeek(a.failed));
+                sh[0] = take ? a.order[q] : 0;
+                sh[1] = take ? 1 : (int)kTeamQuit;
+            } else if (rank == 0) {
+                const int q = keep ? (int)atomicAdd(a.ticket + 1, 1u) : a.nWide;
+                int size = (int)kTeamSolo, sys = 0;
+                if (q < a.nWide) {
                     sys = a.order[q];
-                    const int want = teamWant(a.sys[sys], a.team);
+                    const int want = teamWant(levelRows(a.sys[sys]), a.team);
                     size = 1;
                     for (int k = 0; want > 1 && k < 64; ++k) {  // the members start at about this time
                         const int here = (int)__hip_atomic_load(&a.arrived[xcd], __ATOMIC_RELAXED,
@@ -903,25 +920,32 @@ __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
         const int sys = sh[0], size = sh[1];
         number = (unsigned)sh[2];
         __syncthreads();
-        if (size == (int)kTeamQuit) return;  // the queue is empty
-        if (size == 1) {
+        if (size == (int)kTeamQuit) return;  // the queue is empty: every workgroup ends here
+        if (size == (int)kTeamSolo) {
+            solo = true;
+        } else if (size == 1) {
             solveAlone<VR>(a, sys, red);  // (posted to nobody)
         } else if (rank < size) {
-            TeamComm c{slot, rank, size, (unsigned long long)number << 40, 0, Waits(a.waitLimit, a.failed, a.fail),
-                       &dead};
+            TeamComm c{slot, rank, size, (unsigned long long)number << 40, 0, a, &dead};
             solveInTeam(c, a, sys);
             if (c.broken()) {
-                if (rank == 0 && threadIdx.x == 0) post(number + 1, kTeamQuit, 0);
+                if (threadIdx.x == 0) {
+                    __hip_atomic_store(a.failed, kGroupBroken, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    *a.fail = 1;
+                    if (rank == 0) post(number + 1, kTeamQuit, 0);
+                }
                 return;
             }
         }
     }
 }
 
-__global__ void kResetQueue(unsigned* ticket, unsigned* arrived, GroupStep* failed, TeamSlot* slots, int nSlots) {
+__global__ void kResetQueue(unsigned* ticket, int nWide, unsigned* arrived, GroupStep* failed, TeamSlot* slots,
+                            int nSlots) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t == 0) {
-        *ticket = 0u;
+        ticket[0] = (unsigned)nWide;
+        ticket[1] = ticket[2] = 0u;
         *failed = 0ull;
     }
     if (t < kBatchXcds) arrived[t] = 0u;
@@ -940,6 +964,12 @@ struct unap_hip_batch_s {
     long long total = 0;
     std::vector<BatchSys> sysH;
     std::vector<int> permH;       // global internal -> global external cell
+    std::vector<double> cost;     // a system's time in one workgroup, in arbitrary units
+    std::vector<int> orderH;      // systems, largest work first
+    int team = 0;                 // workgroups a team, as set; 0: chosen
+    int planned = -1;             // the setting that the plan below is for
+    int teamSize = 1, teamWide = 0, teams = 0;
+    DBuf<int> teamOrder;
     DBuf<BatchSys> sys;
     DBuf<int> order;
     DBuf<unsigned> ticket;
@@ -986,24 +1016,29 @@ void launchShape(const BatchArgs& a, int grid, int vr, hipStream_t st) {
     }
 }
 
-// Workgroups a team (launches of 1024 threads): none where no system's average
-// level fills a workgroup; then 8, or 4 where the systems outnumber half the
-// CUs and their leaders would be too few.  ms a solve alone / teams of 4 / of 8
-// (MI355X, random numberings): 96 systems of 8..48 a side 364 / 175 / 141; 24
-// of 10..40 155 / 85 / 61; 300 of 8..40 207 / 143 / 231; 64 of 8..24, levels of
-// up to 920 rows 20.2 / 21.7 / 21.3.  Teams of 16: 206, 67, 425.
-int teamSize(const unap_hip_batch_s& B) {
-    int rows = 0;
-    for (const BatchSys& d : B.sysH) rows = std::max(rows, d.n / std::max(1, std::max(d.nFwd, d.nBwd)));
-    if (rows < 1024) return 1;
-    return 2 * B.nsys <= B.cus ? 8 : 4;
+// The plan for the team size set, made again when another one is.
+void makePlan(unap_hip_batch_s& B, hipStream_t s) {
+    if (B.planned == B.team) return;
+    std::vector<TeamSystem> sys(B.nsys);
+    for (int i = 0; i < B.nsys; ++i) sys[i] = {levelRows(B.sysH[i]), B.cost[i]};
+    const TeamPlan p = planTeams(sys, B.orderH, B.cus, B.team);
+    B.planned = -1;  // (an upload that fails leaves no plan)
+    B.teamOrder.upload(p.order, s);
+    UH_CHECK(hipStreamSynchronize(s));  // the host list dies here
+    B.teamSize = p.size;
+    B.teamWide = p.wide;
+    B.teams = p.teams;
+    B.planned = B.team;
 }
 
 void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIter, int bs, int wgPerCU, int vr) {
     Ctx& c = Ctx::get();
     BatchArgs a;
     a.sys = B.sys.get();
-    a.order = B.order.get();
+    a.team = bs == 1024 ? B.teamSize : 1;
+    a.teams = B.teams;
+    a.nWide = a.team > 1 ? B.teamWide : 0;
+    a.order = a.team > 1 ? B.teamOrder.get() : B.order.get();
     a.nsys = B.nsys;
     a.ticket = B.ticket.get();
     a.rowInfo = B.rowInfo.get();
@@ -1028,15 +1063,14 @@ void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIt
     a.maxIter = maxIter;
     a.perf = B.perf.get();
     const int grid = std::max(1, std::min(B.nsys, B.cus * wgPerCU));
-    a.team = bs == 1024 ? teamSize(B) : 1;
     a.arrived = B.arrived.get();
     a.slots = B.slots.get();
     a.slotsPerXcd = B.cus;
     a.failed = B.failed.get();
     a.fail = const_cast<int*>(c.groupFail);
-    a.waitLimit = c.waitLimit;
+    a.waitLimit = std::min(c.waitLimit, kTeamLimit);
     const int nSlots = (int)B.slots.n;
-    kResetQueue<<<(nSlots + 255) / 256, 256, 0, c.stream>>>(B.ticket.get(), B.arrived.get(), B.failed.get(),
+    kResetQueue<<<(nSlots + 255) / 256, 256, 0, c.stream>>>(B.ticket.get(), a.nWide, B.arrived.get(), B.failed.get(),
                                                             B.slots.get(), nSlots);
     UH_LAUNCHED();
     if (a.team > 1) {
@@ -1086,6 +1120,7 @@ int unap_hip_batch_create(int64_t nsys, const int64_t* cellOff, const int64_t* f
         std::vector<float> tRd[2], tCoef[2];
         std::vector<int> tCol[2];
         std::vector<double> work(nsys);
+        B->cost.resize(nsys);
         for (int64_t s = 0; s < nsys; ++s) {
             const int64_t n = cellOff[s + 1] - cellOff[s], nf = faceOff[s + 1] - faceOff[s];
             if (n <= 0 || nf < 0) throw Error(UNAP_HIP_ERR_ARG, "empty system in batch");
@@ -1200,15 +1235,17 @@ int unap_hip_batch_create(int64_t nsys, const int64_t* cellOff, const int64_t* f
             std::vector<double> dd;
             fillDiag<double>(L, A, dd);
             diagAll.insert(diagAll.end(), dd.begin(), dd.end());
-            work[s] = (double)(n + 2 * nf) * std::cbrt((double)n) * (dic ? 1.0 : 2.0);
+            B->cost[s] = (double)(n + 2 * nf) * std::cbrt((double)n);
+            work[s] = B->cost[s] * (dic ? 1.0 : 2.0);
         }
         B->total = cellOff[nsys];
-        std::vector<int> ord(nsys);
+        std::vector<int>& ord = B->orderH;
+        ord.resize(nsys);
         std::iota(ord.begin(), ord.end(), 0);
         std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return work[a] > work[b]; });
         B->sys.upload(B->sysH, c.stream);
         B->order.upload(ord, c.stream);
-        B->ticket.alloc(1);
+        B->ticket.alloc(3);
         B->rowInfo.upload(infoAll, c.stream);
         if (ellColAll.empty()) {  // diagonal systems only: keep the pointers valid
             ellColAll.push_back(0);
@@ -1273,6 +1310,7 @@ int unap_hip_batch_solve(unap_hip_batch B, double* x, const double* b, int where
         }
         launchRows(BGather<double, double>{B->perm.get(), bs, B->b.get()}, (int)T);
         launchRows(BGather<double, double>{B->perm.get(), xs, B->x.get()}, (int)T);
+        makePlan(*B, c.stream);
         // x0 is kept to restart from it while tuning
         DBuf<double> x0(T);
         UH_CHECK(hipMemcpyAsync(x0.get(), B->x.get(), sizeof(double) * T, hipMemcpyDeviceToDevice, c.stream));
@@ -1346,6 +1384,24 @@ int unap_hip_batch_config(unap_hip_batch B, int64_t* block_size, int64_t* wg_per
         if (block_size) *block_size = B->blockSize;
         if (wg_per_cu) *wg_per_cu = B->wgPerCU;
         if (rows_per_wavefront) *rows_per_wavefront = 64 * B->rowsPerThread;
+    });
+}
+
+int unap_hip_batch_set_team(unap_hip_batch B, int64_t workgroups) {
+    return bguard([&] {
+        if (!B) throw Error(UNAP_HIP_ERR_ARG, "null argument");
+        if (workgroups < 0 || workgroups > kTeamMax)
+            throw Error(UNAP_HIP_ERR_ARG, "a team holds 1 to 8 workgroups (0: chosen)");
+        B->team = (int)workgroups;
+    });
+}
+
+int unap_hip_batch_team(unap_hip_batch B, int64_t* workgroups, int64_t* systems) {
+    return bguard([&] {
+        if (!B) throw Error(UNAP_HIP_ERR_ARG, "null argument");
+        const bool on = B->blockSize == 1024 && B->teamSize > 1;
+        if (workgroups) *workgroups = on ? B->teamSize : 1;
+        if (systems) *systems = on ? B->teamWide : 0;
     });
 }
 

@@ -115,6 +115,8 @@ SIGNATURES = {
                                             ctypes.POINTER(Perf)]),
     "unap_hip_batch_last_ms": (ctypes.c_int, [_vp, _f64p]),
     "unap_hip_batch_config": (ctypes.c_int, [_vp, _i64p, _i64p, _i64p]),
+    "unap_hip_batch_team": (ctypes.c_int, [_vp, _i64p, _i64p]),
+    "unap_hip_batch_set_team": (ctypes.c_int, [_vp, ctypes.c_int64]),
     "unap_hip_batch_set_config": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]),
 }
 
@@ -723,6 +725,16 @@ class Batch:
         bs, wg, rw = _i64(), _i64(), _i64()
         _check(lib().unap_hip_batch_config(self.h, ctypes.byref(bs), ctypes.byref(wg), ctypes.byref(rw)))
         return bs.value, wg.value, rw.value
+
+    def set_team(self, workgroups=0):
+        """Workgroups that share a large system at 1024 threads (1: none do; 0: chosen)."""
+        _check(lib().unap_hip_batch_set_team(self.h, workgroups))
+
+    def team(self):
+        """(workgroups a team, systems that teams take) of the last solve; (1, 0): no teams."""
+        size, wide = _i64(), _i64()
+        _check(lib().unap_hip_batch_team(self.h, ctypes.byref(size), ctypes.byref(wide)))
+        return size.value, wide.value
 
     def set_config(self, block_size, wg_per_cu, rows_per_wavefront=256):
         """Fix the launch shape (the autotuner then does not run)."""
