@@ -397,7 +397,8 @@ int unap_hip_batch_config(unap_hip_batch B, int64_t* block_size, int64_t* wg_per
                           int64_t* rows_per_wavefront);
 /* Set the launch shape and skip the autotuner: block_size 256, 512 or 1024,
    wg_per_cu >= 1 with block_size * wg_per_cu <= 2048, rows_per_wavefront 64,
-   128 or 256 (results do not depend on it). */
+   128 or 256 (results do not depend on it).  A CU runs one workgroup of 1024
+   threads at a time: wg_per_cu makes no difference there. */
 int unap_hip_batch_set_config(unap_hip_batch B, int64_t block_size, int64_t wg_per_cu,
                               int64_t rows_per_wavefront);
 /* Workgroups on one XCD that share a large system, in launches of 1024

@@ -62,3 +62,16 @@ def test_refused_sizes():
     for size in (-1, 9):
         with pytest.raises(hip.UnapHipError):
             B.set_team(size)
+
+
+def test_tuner_times_a_launch_of_teams_once():
+    systems = [_box(d, k, i) for i, (d, k) in enumerate(LARGE[:2])]
+    B = hip.Batch(systems, ["PCG" if s.symmetric else "PBiCGStab" for s in systems])
+    x, _ = B.solve(np.concatenate([s.b for s in systems]), max_iter=20)
+    bs, wg, _ = B.config()
+    assert bs in (256, 512, 1024) and (bs < 1024 or wg == 1)
+    B.set_config(1024, 2, 256)  # accepted, and the same as (1024, 1)
+    y, _ = B.solve(np.concatenate([s.b for s in systems]), max_iter=20)
+    assert B.config() == (1024, 2, 256) and B.team()[0] > 1
+    B.set_config(1024, 1, 256)
+    assert np.array_equal(y, B.solve(np.concatenate([s.b for s in systems]), max_iter=20)[0])

@@ -1062,6 +1062,8 @@ void launchBatch(unap_hip_batch_s& B, double relTol, double tol, long long maxIt
     a.tol = tol;
     a.maxIter = maxIter;
     a.perf = B.perf.get();
+    // (workgroups of 1024 threads fill a CU's registers: a second one a CU
+    // starts when the first has found the queue empty.  Teams launch one a CU.)
     const int grid = std::max(1, std::min(B.nsys, B.cus * wgPerCU));
     a.arrived = B.arrived.get();
     a.slots = B.slots.get();
@@ -1337,6 +1339,7 @@ int unap_hip_batch_solve(unap_hip_batch B, double* x, const double* b, int where
             for (int bsz : {256, 512, 1024})
                 for (int wg : {1, 2, 4}) {
                     if (bsz * wg > 2048) continue;
+                    if (bsz == 1024 && wg > 1 && B->teamSize > 1) continue;  // the same launch
                     const double ms = timed(bsz, wg, 4);
                     if (ms < best) {
                         best = ms;
