@@ -308,6 +308,10 @@ int unap_hip_solver_last_ms(unap_hip_solver S, double* ms);
 #define UNAP_HIP_KERNEL_COPY 8       /* y = x, a plain copy (achievable-bandwidth yardstick) */
 int unap_hip_profile_kernel(unap_hip_ldu A, int kernel, int precision, int64_t reps, double* avg_ms,
                             double* bytes);
+/* How the matrix's sweeps run, by the size of its levels: *xcds 0: a launch a
+   level; 1 or 8: one launch, by the workgroups of so many XCDs.  kernel: GS, or
+   DIC (DIC and DILU alike). */
+int unap_hip_ldu_sweep_xcds(unap_hip_ldu A, int kernel, int precision, int64_t* xcds);
 /* No counterpart: the setup built on the device (cell orders, sweep
    schedules, SELL-32 layout of each order mode; the agglomeration's pairing
    lists) against the same structures built on the host, for this matrix.

@@ -205,11 +205,15 @@ GroupSpan groupSpan(const DevMatrix<T>& M, size_t levels, double bytesALevel, do
 }
 template <typename T>
 GroupSpan groupGsSpan(const DevMatrix<T>& M) {
+    if (M.gsTab.refused) return GroupSpan::none;
     const size_t nl = M.fwdStartH.size() - 1;
     return groupSpan(M, nl, 16.0 * GroupPack<T>::kGs * M.gsLanes() * M.n / (double)nl, kGroupGsOne, kGroupGsAll);
 }
+// (DIC on asymmetric storage, with its second coefficient array, runs level by
+// level)
 template <typename T>
 GroupSpan groupLuSpan(const DevMatrix<T>& M) {
+    if (M.luTab.refused || M.valU.p) return GroupSpan::none;
     const size_t nl = M.fwdStartH.size() - 1;
     return groupSpan(M, nl + M.bwdStartH.size() - 1, 16.0 * GroupPack<T>::kLu * M.n / (double)nl, kGroupLuOne,
                      kGroupLuAll);
@@ -270,9 +274,8 @@ void luSweeps(DevMatrix<T>& M, bool dic, TV* w, const TV* r, const TV* rD, Skip 
     if (!M.sweepable) throw Error(-3, "DIC/DILU needs faces sorted by owner with owner < neighbour");
     const DMat<T> Av = dic ? M.viewU() : M.view();
     if constexpr (std::is_same<T, TV>::value) {
-        // (DIC on asymmetric storage, with its second coefficient array, and
-        // callers without the position-ordered rD run level by level)
-        const GroupSpan span = M.valU.p || !rDpos ? GroupSpan::none : groupLuSpan(M);
+        // (callers without the position-ordered rD run level by level)
+        const GroupSpan span = rDpos ? groupLuSpan(M) : GroupSpan::none;
         hipStream_t s = Ctx::get().stream;
         if (const GroupTab* t = span != GroupSpan::none ? M.luTable(s) : nullptr) {
             const GroupLu<T> g{Av, M.bwdView(s), t->tab.get(), t->grp0.get(), M.fwdStart.get(), M.bwdStart.get(),

@@ -1809,6 +1809,21 @@ int unap_hip_setup_self_check(unap_hip_ldu A, const double* weights, int64_t* mi
     });
 }
 
+int unap_hip_ldu_sweep_xcds(unap_hip_ldu A, int kernel, int precision, int64_t* xcds) {
+    return guard([&] {
+        checkLduReady(A);
+        need(xcds != nullptr, "null argument");
+        need(kernel == UNAP_HIP_KERNEL_GS || kernel == UNAP_HIP_KERNEL_DIC, "kernel is GS or DIC");
+        need(precision == 64 || precision == 32, "precision is 64 or 32");
+        auto span = [&](const auto& M) {
+            if (!M.sweepable) throw Error(UNAP_HIP_ERR_FACE_ORDER, "the faces are not owner-sorted");
+            return kernel == UNAP_HIP_KERNEL_GS ? groupGsSpan(M) : groupLuSpan(M);
+        };
+        const GroupSpan s = precision == 64 ? span(A->o.dev64(ORDER_SWEEP)) : span(A->o.dev32(ORDER_SWEEP));
+        *xcds = s == GroupSpan::none ? 0 : (s == GroupSpan::one ? 1 : kXcds);
+    });
+}
+
 int unap_hip_profile_kernel(unap_hip_ldu A, int kernel, int precision, int64_t reps, double* avgMs, double* bytes) {
     return guard([&] {
         need(A && avgMs && bytes, "null argument");

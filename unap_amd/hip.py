@@ -73,6 +73,7 @@ SIGNATURES = {
     "unap_hip_ldu_read_hypre": (ctypes.c_int, [ctypes.c_char_p, ctypes.POINTER(_vp)]),
     "unap_hip_vector_read_hypre": (ctypes.c_int, [ctypes.c_char_p, _i64, _f64p]),
     "unap_hip_rcm_order": (ctypes.c_int, [_i64, _i64, _i64p, _i64p, _i64p]),
+    "unap_hip_ldu_sweep_xcds": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int, _i64p]),
     "unap_hip_setup_self_check": (ctypes.c_int, [_vp, _f64p, _i64p]),
     "unap_hip_ldu_renumber": (ctypes.c_int, [_i64, _i64, _i64p, _i64p, _i64p, _f64p, _f64p, _f64p,
                                              _i64p, _i64p, _i64p, _f64p, _f64p, _f64p]),
@@ -291,6 +292,13 @@ def read_vector_hypre(path, n):
     out = np.empty(n)
     _check(lib().unap_hip_vector_read_hypre(os.fsencode(path), n, _p(out)))
     return out
+
+
+def sweep_xcds(A, kind, precision=64):
+    """XCDs whose workgroups run a sweep ("GS" or "DIC") of A in one launch; 0: a launch a level."""
+    v = _i64()
+    _check(lib().unap_hip_ldu_sweep_xcds(A.h, {"GS": 3, "DIC": 4}[kind], precision, ctypes.byref(v)))
+    return v.value
 
 
 def setup_self_check(A, weights=None):
