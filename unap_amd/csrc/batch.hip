@@ -510,8 +510,10 @@ __device__ void batchBiCG(const BatchArgs& a, const SysView& s, int off, unap_hi
 // wavefronts' sums are added in their order.  So every result is bitwise that
 // of one workgroup, whatever the team's size.
 //
-// A team's leader takes systems from the queue and posts them to the members
-// that have started; it never waits for a workgroup that may not be running.
+// A team's leader takes the teams' systems from their queue and posts them to
+// the members that have started; it never waits for a workgroup that may not be
+// running.  When that queue is empty it ends the team, and each of its
+// workgroups takes other systems alone.
 // A barrier that never ends all the same (a fault in this scheme) gives up
 // after some tenths of a second.  The workgroup leaves its solve at the end of
 // the iteration, its team's others give up as well, a leader ends its team and
@@ -920,7 +922,7 @@ __global__ void __launch_bounds__(BS) kBatchTeams(BatchArgs a) {
         const int sys = sh[0], size = sh[1];
         number = (unsigned)sh[2];
         __syncthreads();
-        if (size == (int)kTeamQuit) return;  // the queue is empty: every workgroup ends here
+        if (size == (int)kTeamQuit) return;  // the queues are empty (or the launch is broken)
         if (size == (int)kTeamSolo) {
             solo = true;
         } else if (size == 1) {

@@ -137,7 +137,10 @@ struct CoarseLocal {
     // entries) in that order.  LDS loads go kLocalBatch at a time (columns
     // and coefficients, then the gathers), positions past the end re-reading
     // the batch's first entry, so a row waits on two LDS round trips a batch
-    // rather than two an entry.
+    // rather than two an entry.  Four: the sweeps' rows are held (HeldRow), and
+    // what is left, the products and the entries past the held ones, is slower
+    // in batches of eight (PCG + AMG solves: 120^3 Chebyshev 68.6 against 65.0
+    // ms, 128^3 Gauss-Seidel 250 against 244).
     static constexpr int kLocalBatch = 4;
     template <int Op>  // 0: acc + v x;  1: acc - (rd v) x
     __device__ __forceinline__ double run(int k0, int n, int step, double acc, double rd, const double* x) const {
@@ -341,10 +344,10 @@ __device__ __forceinline__ void heldSweep(const CoarseLocal& m, int nRows, int n
 
 // kCoarsePCG with the matrix, rD, the schedule and the vectors in LDS, and
 // both sweeps' rows in registers (one row of each sweep a thread; a
-// level's rows past the threads run from LDS): 18 iterations of 60 levels on 556 rows took 1345 us with the
-// sweeps' matrix read from LDS by 256 threads (a level's row index, bounds,
-// entries and gathers one after the other), 613 us so; a 57-row one 300 and
-// 120 us.  What is left is the chain of a level: barrier, gathers,
+// level's rows past the threads run from LDS): 18 iterations of 60 levels on
+// 556 rows took 1345 us with the sweeps' matrix read from LDS by 256 threads (a
+// level's row index, bounds, entries and gathers one after the other), 613 us
+// so; a 57-row one 300 and 120 us.  What is left is the chain of a level: barrier, gathers,
 // subtractions, and the entries past Cap, which come from LDS.
 constexpr int kCoarseSum = 256;  // threads of the reductions' tree
 template <int Threads, int Cap>

@@ -18,9 +18,10 @@
 // workgroup that has no place on the device, and the work is split by the
 // number that registered.  A wait that never ends all the same (a fault in
 // this scheme) gives up after some seconds.  That is reported to the host, and
-// from then on nothing waits: the workgroup that gave up goes through its
-// remaining steps without, the others see the failure in their waits, and the
-// launches queued behind leave at once, until the host has reported the error.
+// from then on nothing waits long: the workgroup that gave up goes through its
+// remaining steps with a poll a wait, the others see the failure in theirs, and
+// the launches queued behind leave at once, until the host has reported the
+// error.
 //
 // Visibility.  Values that cross workgroups (the swept vector, the flags) are
 // read with agent-scope loads, which pass the CU's own cache; the group on one
@@ -44,7 +45,8 @@ constexpr int kWaitLook = 1 << 14;       // polls between looks at the failure w
 // their own; words polled together share one.  The words of the list are zero
 // between launches.  The steps are never reset: they count on from launch to
 // launch (epoch), because an XCD's own flags stay dirty in its L2, and a reset
-// from another XCD would be undone when they are written back.
+// from another XCD would be undone when they are written back.  What a word
+// left from earlier launches may hold: group_steps.hpp.
 template <typename W>
 struct GroupWords {
     W flag[kXcds][kGroupPerXcd];    // step reached, by workgroup
