@@ -55,8 +55,8 @@ int unap_hip_set_reduction_order(int order);
 
 /* Polls that a workgroup of a sweep or a batch's team waits for another before
    the call ends in UNAP_HIP_ERR_INTERNAL: 0 to 2^23, the default (seconds).
-   Applies to kernels launched or captured from then on.  No reference
-   counterpart; a wait that long is a fault of the device or of the library. */
+   No reference counterpart; a wait that long is a fault of the device or of
+   the library. */
 int unap_hip_set_wait_limit(int64_t polls);
 
 /* Solver iterations from the second on replayed from a HIP graph of one

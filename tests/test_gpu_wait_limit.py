@@ -35,6 +35,24 @@ def test_sweeps(oracle, no_polls, dims):
         assert np.array_equal(P.apply(s.b), O.precond("DILU", s.b)[0])
 
 
+@pytest.mark.parametrize("graphs", [True, False])
+def test_solves(oracle, no_polls, graphs):
+    s = meshgen.box_system(40, 41, 39, meshgen.POISSON_LOGUNIF, -3.0, 0.0, 1e-6, 5)
+    A = hip.LduMatrix.from_system(s)
+    hip.set_graph_replay(graphs)
+    try:
+        for pre, amg in (("DIC", None), ("AMG", hip.amg_params(smoother=1, n_cells_coarsest=100, n_vcycles=1))):
+            S = hip.Solver("PCG", hip.Precond(A, pre, amg=amg), rel_tol=1e-8, max_iter=300)
+            x, p = S.solve(A, s.b)
+            assert p["converged"]
+            for _ in range(2):
+                no_polls(lambda: S.solve(A, s.b))
+                y, q = S.solve(A, s.b)
+                assert np.array_equal(x, y) and p["nIterations"] == q["nIterations"]
+    finally:
+        hip.set_graph_replay(True)
+
+
 def test_teams(no_polls):
     systems = [meshgen.box_system(33, 31, 29, meshgen.POISSON_LOGUNIF, -3.0, 0.0, 1e-6, 1),
                meshgen.box_system(30, 27, 35, meshgen.CONVDIFF, 5.0, 0.0, 1e-3, 2)]

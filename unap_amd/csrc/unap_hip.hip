@@ -1943,7 +1943,8 @@ int unap_hip_solver_solve(unap_hip_solver S, unap_hip_ldu A, double* x, const do
         d.key = {L.id, (unsigned long long)L.coeffGen, (unsigned long long)L.topoGen,
                  (unsigned long long)(uintptr_t)o.P, (unsigned long long)o.type,
                  (unsigned long long)c.serialReductions, (unsigned long long)(uintptr_t)S->bufs.x.get(),
-                 (unsigned long long)(uintptr_t)S->bufs.hist.get(), (unsigned long long)(uintptr_t)o.mgH.get()};
+                 (unsigned long long)(uintptr_t)S->bufs.hist.get(), (unsigned long long)(uintptr_t)o.mgH.get(),
+                 (unsigned long long)c.waitLimit};
         switch (o.type) {
             case UNAP_HIP_SOLVER_PCG: d.pcg(); break;
             case UNAP_HIP_SOLVER_PBICGSTAB: d.bicg(); break;
